@@ -327,6 +327,8 @@ void ffvhc_ctx_destroy(ffvhc_ctx* c) {
   (void)hipFree(c->dcuni);
   (void)hipFree(c->dctab);
   (void)hipFree(c->dctrec);
+  (void)hipFree(c->drows_uni);
+  (void)hipFree(c->drows);
   (void)hipFree(c->dcut);
   (void)hipFree(c->dflag);
   (void)hipFree(c->dcid);

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cfloat>
+#include <type_traits>
 
 #include "device.h"
 #include "ghost.h"
@@ -102,6 +103,50 @@ __device__ inline void stage_block(T* s, const T* __restrict__ x, const T* __res
   }
 }
 
+
+// Stencil position classes: a cell's class is (cx, cy, cz), each 0 on the block's low face layer,
+// 2 on its high one and 1 inside (27 classes, index cx + 3 cy + 9 cz); the representative of a class
+// is its lowest-index cell.
+__device__ inline int stencil_class1(int i) { return i == 0 ? 0 : i == NB - 1 ? 2 : 1; }
+__device__ inline int stencil_rep1(int c) { return c == 0 ? 0 : c == 2 ? NB - 1 : 1; }
+
+// The three rows (k = 0, inside, k = NB - 1) of the column (tx, ty) of block `slot`
+template <class T>
+__device__ inline const T* class_column(const T* __restrict__ tab, int slot, int tx, int ty) {
+  return tab + ((size_t)slot * 27 + stencil_class1(tx) + 3 * stencil_class1(ty)) * 8;
+}
+
+// Bands of one (i, j) column of a block.  CLS: the block is class-uniform, so its bands come from the
+// column's three class rows, held in registers; else from the per-cell arrays.
+template <class T, bool CLS>
+struct ColumnBands {
+  T lo[7], in[7], hi[7];
+  __device__ ColumnBands(const ClassRows<T>& R, int slot, int tx, int ty) {
+    if constexpr (CLS) {
+      const T* tr = class_column(R.tab, slot, tx, ty);
+#pragma unroll
+      for (int q = 0; q < 7; q++) {
+        lo[q] = tr[q];
+        in[q] = tr[9 * 8 + q];
+        hi[q] = tr[18 * 8 + q];
+      }
+    }
+  }
+  // coefficient q of plane k (a constant once unrolled) at cell g
+  __device__ T operator()(const Coef7<T>& A, int q, int k, size_t g) const {
+    if constexpr (CLS) return k == 0 ? lo[q] : k == NB - 1 ? hi[q] : in[q];
+    return A.p[q][g];
+  }
+};
+
+// f(true_type) for a class-uniform block, f(false_type) else (uniform over the workgroup)
+template <class T, class F>
+__device__ inline void by_class(const ClassRows<T>& R, int slot, const F& f) {
+  if (R.uni && R.uni[slot])
+    f(std::true_type{});
+  else
+    f(std::false_type{});
+}
 
 __device__ inline void converged(SolveState& s, double rr, int count) {
   // FFVILS.h:24-47 IsConverged

@@ -32,7 +32,7 @@ void launch_ghost_pull(hipStream_t sm, const int* active, int nact, const DevBlo
 template <class T>
 void launch_rbgs_iter(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                       SolveState* st, Coef7<T> A, const T* b, const T* xin, T* xout, const T* hin, T* hout,
-                      double* part, size_t nslots, int n, int bcg, int mode = 0);
+                      double* part, size_t nslots, int n, int bcg, int mode = 0, ClassRows<T> R = ClassRows<T>());
 template <class T>
 void launch_shift_push(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                        const SolveState* st, T* x, const T* hin, T* hout, int bcg);
@@ -48,20 +48,24 @@ void launch_copy(hipStream_t sm, const int* active, int nact, T* y, T* hy, const
 
 template <class T>
 void launch_cg_init(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs, SolveState* st,
-                    Coef7<T> A, const T* b, const T* x, const T* hx, T* r, double* part, size_t nslots);
+                    Coef7<T> A, const T* b, const T* x, const T* hx, T* r, double* part, size_t nslots,
+                    ClassRows<T> R = ClassRows<T>());
 template <class T>
 void launch_cg_p(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
-                 const SolveState* st, Coef7<T> A, const T* r, T* p, T* hp, int count, int bcg);
+                 const SolveState* st, Coef7<T> A, const T* r, T* p, T* hp, int count, int bcg,
+                 ClassRows<T> R = ClassRows<T>());
 template <class T>
 void launch_cg_q(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs, SolveState* st,
-                 Coef7<T> A, const T* p, const T* hp, T* q, double* part);
+                 Coef7<T> A, const T* p, const T* hp, T* q, double* part, ClassRows<T> R = ClassRows<T>());
 template <class T>
 void launch_cg_xr(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs, SolveState* st,
-                  Coef7<T> A, T* x, T* r, const T* p, const T* q, double* part, size_t nslots, int count);
+                  Coef7<T> A, T* x, T* r, const T* p, const T* q, double* part, size_t nslots, int count,
+                  ClassRows<T> R = ClassRows<T>());
 template <class T>
 void launch_bicgstab_init(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                           SolveState* st, Coef7<T> A, const T* b, const T* x, const T* hx, BiVecs<T> V, double* part,
-                          size_t nslots, bool hash_r0 = false, double* bsr = nullptr);
+                          size_t nslots, bool hash_r0 = false, double* bsr = nullptr,
+                          ClassRows<T> R = ClassRows<T>());
 // Precision options of an FP64 BiCGSTAB: A32 = FP32 copy of the matrix for the matvecs and the
 // Jacobi preconditioner (widened to FP64 on load); gs = block red-black GS preconditioner with
 // an FP32 matrix and FP32 arithmetic, an FP32 matrix and FP64 arithmetic, all FP64, or the
@@ -98,7 +102,8 @@ struct BiOpts {
 template <class T>
 void launch_bicgstab_iter(hipStream_t sm, const int* active, int nact, const int* caseact, int ncase,
                           const DevBlock* blk, const DevCase* cs, SolveState* st, Coef7<T> A, T* x, BiVecs<T> V,
-                          double* part, size_t nslots, int count, int mask = 31, const BiOpts& o = BiOpts());
+                          double* part, size_t nslots, int count, int mask = 31, const BiOpts& o = BiOpts(),
+                          ClassRows<T> R = ClassRows<T>());
 template <class T>
 void launch_bicgstab_reanchor(hipStream_t sm, const int* active, int nact, const DevBlock* blk,
                               const SolveState* gate, BiVecs<T> V, double* part, size_t nslots);
@@ -120,6 +125,9 @@ void launch_gs_pack(hipStream_t sm, const int* active, int nact, Coef7<double> A
 // its 27 class rows: FP32 bands tab[slot][27][8] and preconditioner records trec[slot][27]
 void launch_stencil_classes(hipStream_t sm, const int* active, int nact, Coef7<double> A, int* uniform, float* tab,
                             uint4* trec);
+// the flags and the 27 rows in the matrix's own precision (the reference solvers)
+template <class T>
+void launch_class_rows(hipStream_t sm, const int* active, int nact, Coef7<T> A, int* uniform, T* tab);
 // coarse operator rows (25 doubles per slot), dense Gauss-Jordan inversion, FP32 copy, apply
 void launch_coarse_rows(hipStream_t sm, const int* active, int nact, const DevBlock* blk, Coef7<double> A,
                         double* rows);

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(BI_NT) void bi_init_kernel(const int* __restrict__ 
                                                         Coef7<T> A, const T* __restrict__ bv, const T* __restrict__ x,
                                                         const T* __restrict__ hx, BiVecs<T> V,
                                                         double* __restrict__ part, size_t nslots,
-                                                        double* __restrict__ bsr) {
+                                                        double* __restrict__ bsr, ClassRows<T> R) {
   __shared__ T s[LP * LP * LP];
   __shared__ double red[BI_NT / 64];
   const int slot = active[blockIdx.x];
@@ -52,38 +52,41 @@ __global__ __launch_bounds__(BI_NT) void bi_init_kernel(const int* __restrict__ 
   const uint32_t local = (uint32_t)(slot - cs[c].slot_begin);
   constexpr int KB = Batch<T>::K;
   double bb = 0.0, rr1 = 0.0, rs = 0.0;
+  by_class(R, slot, [&](auto cls) {
+    const ColumnBands<T, decltype(cls)::value> W(R, slot, tx, ty);
 #pragma unroll
-  for (int k0 = 0; k0 < NB; k0 += KB) {
-    T a[KB][7], b0[KB];
+    for (int k0 = 0; k0 < NB; k0 += KB) {
+      T a[KB][7], b0[KB];
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
 #pragma unroll
-      for (int q = 0; q < 7; q++) a[kk][q] = A.p[q][g];
-      b0[kk] = bv[g];
-    }
-    if (k0 == 0) {
-      stage_block<T, BI_NT>(s, x, hx, slot);
-      __syncthreads();
-    }
+        for (int q = 0; q < 7; q++) a[kk][q] = W(A, q, k0 + kk, g);
+        b0[kk] = bv[g];
+      }
+      if (k0 == 0) {
+        stage_block<T, BI_NT>(s, x, hx, slot);
+        __syncthreads();
+      }
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      const int li = lds(tx, ty, k0 + kk);
-      const T r = b0[kk] - a[kk][1] * s[li - 1] - a[kk][2] * s[li + 1] - a[kk][3] * s[li - LP] -
-                  a[kk][4] * s[li + LP] - a[kk][5] * s[li - LP * LP] - a[kk][6] * s[li + LP * LP] -
-                  a[kk][0] * s[li];
-      V.r[g] = r;
-      rs += (double)r;
-      bb += (double)b0[kk] * (double)b0[kk];
-      if (HR) {
-        rr1 += (double)r * (double)shadow_value(local, (uint32_t)(g - base));
-      } else {
-        V.r0[g] = r;
-        rr1 += (double)r * (double)r;
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        const int li = lds(tx, ty, k0 + kk);
+        const T r = b0[kk] - a[kk][1] * s[li - 1] - a[kk][2] * s[li + 1] - a[kk][3] * s[li - LP] -
+                    a[kk][4] * s[li + LP] - a[kk][5] * s[li - LP * LP] - a[kk][6] * s[li + LP * LP] -
+                    a[kk][0] * s[li];
+        V.r[g] = r;
+        rs += (double)r;
+        bb += (double)b0[kk] * (double)b0[kk];
+        if (HR) {
+          rr1 += (double)r * (double)shadow_value(local, (uint32_t)(g - base));
+        } else {
+          V.r0[g] = r;
+          rr1 += (double)r * (double)r;
+        }
       }
     }
-  }
+  });
   double sb = block_sum<BI_NT>(bb, red);
   double sr = block_sum<BI_NT>(rr1, red);
   if (t == 0) {
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(BI_NT) void bi_precond_kernel(const int* __restrict
                                                            const DevBlock* __restrict__ blk,
                                                            const DevCase* __restrict__ cs,
                                                            const SolveState* __restrict__ st, Coef7<TA> A, BiVecs<T> V,
-                                                           int count) {
+                                                           int count, ClassRows<TA> R) {
   __shared__ T s[LP * LP * LP];
   const int slot = active[blockIdx.x];
   const DevBlock& B = blk[slot];
@@ -117,39 +120,44 @@ __global__ __launch_bounds__(BI_NT) void bi_precond_kernel(const int* __restrict
   // arguments); FIN_BI_XR of the previous iteration stored it in iter
   const bool first = (count > 0 ? count : st[c].iter + 1) == 1 || st[c].restart;
   constexpr int KB = Batch<T>::K;
+  by_class(R, slot, [&](auto cls) {
+    constexpr bool CLS = decltype(cls)::value;
+    const TA* tr = CLS ? class_column(R.tab, slot, tx, ty) : nullptr;
+    const T alo = CLS ? (T)tr[0] : (T)0, ain = CLS ? (T)tr[9 * 8] : (T)0, ahi = CLS ? (T)tr[18 * 8] : (T)0;
 #pragma unroll
-  for (int k0 = 0; k0 < NB; k0 += KB) {
-    T rv[KB], pv[KB], qv[KB], ap[KB];
+    for (int k0 = 0; k0 < NB; k0 += KB) {
+      T rv[KB], pv[KB], qv[KB], ap[KB];
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      rv[kk] = V.r[g];
-      ap[kk] = (T)A.p[0][g];
-      if (MODE == 1 || !first) qv[kk] = V.q[g];
-      if (MODE == 0 && !first) pv[kk] = V.p[g];
-    }
-#pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      T v;
-      if (MODE == 0) {
-        if (first) {
-          v = rv[kk];
-        } else {
-          const T tmp = pv[kk] + ng * qv[kk];  // AXPY(p, q_, -gamma)
-          v = rv[kk] + beta * tmp;             // XPAY(p, r, beta)
-        }
-        V.p[g] = v;
-      } else {
-        v = na * qv[kk] + rv[kk];  // AXPYZ(s, q_, r, -alpha)
-        V.s[g] = v;
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        rv[kk] = V.r[g];
+        ap[kk] = CLS ? (k0 + kk == 0 ? alo : k0 + kk == NB - 1 ? ahi : ain) : (T)A.p[0][g];
+        if (MODE == 1 || !first) qv[kk] = V.q[g];
+        if (MODE == 0 && !first) pv[kk] = V.p[g];
       }
-      const T m = omega * (v / ap[kk]);
-      if (MODE == 0) V.pp[g] = m;
-      else V.ss[g] = m;
-      s[lds(tx, ty, k0 + kk)] = m;
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        T v;
+        if (MODE == 0) {
+          if (first) {
+            v = rv[kk];
+          } else {
+            const T tmp = pv[kk] + ng * qv[kk];  // AXPY(p, q_, -gamma)
+            v = rv[kk] + beta * tmp;             // XPAY(p, r, beta)
+          }
+          V.p[g] = v;
+        } else {
+          v = na * qv[kk] + rv[kk];  // AXPYZ(s, q_, r, -alpha)
+          V.s[g] = v;
+        }
+        const T m = omega * (v / ap[kk]);
+        if (MODE == 0) V.pp[g] = m;
+        else V.ss[g] = m;
+        s[lds(tx, ty, k0 + kk)] = m;
+      }
     }
-  }
+  });
   __syncthreads();
   T* h = MODE == 0 ? V.hpp : V.hss;
   push_halo<T, BI_NT>(B, cs[c], BC_NULL, slot, [&](int i, int j, int k) { return s[lds(i, j, k)]; }, h, h);
@@ -295,9 +303,6 @@ void launch_gs_pack(hipStream_t sm, const int* active, int nact, Coef7<double> A
 // and level interfaces (those change the coefficients of a whole face layer alike).  For such a
 // block the 27 rows -- as FP32 bands (8 floats each, the eighth unused) and as preconditioner
 // records -- stand for the per-cell arrays, bit for bit.
-__device__ inline int stencil_class1(int i) { return i == 0 ? 0 : i == NB - 1 ? 2 : 1; }
-__device__ inline int stencil_rep1(int c) { return c == 0 ? 0 : c == 2 ? NB - 1 : 1; }
-
 __global__ __launch_bounds__(256) void stencil_class_kernel(const int* __restrict__ active, Coef7<double> A,
                                                             int* __restrict__ uniform, float* __restrict__ tab,
                                                             uint4* __restrict__ trec) {
@@ -329,6 +334,51 @@ void launch_stencil_classes(hipStream_t sm, const int* active, int nact, Coef7<d
                             uint4* trec) {
   if (nact) hipLaunchKernelGGL(stencil_class_kernel, dim3(nact), dim3(256), 0, sm, active, A, uniform, tab, trec);
 }
+
+// The same flags and the 27 rows in the matrix's own precision, for the reference solvers (no FP32
+// copy, no records).  Bound by the one pass over the seven bands: the representative rows wait in
+// LDS and the difference is gathered bitwise, so no load waits on a comparison.
+template <class T>
+__global__ __launch_bounds__(256) void class_rows_kernel(const int* __restrict__ active, Coef7<T> A,
+                                                         int* __restrict__ uniform, T* __restrict__ tab) {
+  using Bits = std::conditional_t<sizeof(T) == 8, unsigned long long, unsigned int>;
+  __shared__ T rep[27 * 8];
+  const int slot = active[blockIdx.x];
+  const size_t base = (size_t)slot * NC;
+  const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
+  if (t < 27 * 8) {
+    const int row = t >> 3, q = t & 7;
+    const size_t r = base + stencil_rep1(row % 3) + NB * (stencil_rep1((row / 3) % 3) + NB * stencil_rep1(row / 9));
+    T v = 0;
+#pragma unroll
+    for (int b = 0; b < 7; b++)
+      if (b == q) v = A.p[b][r];
+    rep[t] = v;
+    tab[(size_t)slot * 27 * 8 + t] = v;
+  }
+  __syncthreads();
+  const T* const mine = rep + (stencil_class1(tx) + 3 * stencil_class1(ty)) * 8;
+  Bits diff = 0;
+#pragma unroll
+  for (int q = 0; q < 7; q++) {
+    const T* const b = A.p[q] + base + tx + NB * ty;
+    T v[NB];
+#pragma unroll
+    for (int k = 0; k < NB; k++) v[k] = b[NF * k];
+#pragma unroll
+    for (int k = 0; k < NB; k++)
+      diff |= __builtin_bit_cast(Bits, v[k]) ^ __builtin_bit_cast(Bits, mine[stencil_class1(k) * 9 * 8 + q]);
+  }
+  const int all = __syncthreads_and(diff == 0 ? 1 : 0);
+  if (t == 0) uniform[slot] = all;
+}
+
+template <class T>
+void launch_class_rows(hipStream_t sm, const int* active, int nact, Coef7<T> A, int* uniform, T* tab) {
+  if (nact) hipLaunchKernelGGL(class_rows_kernel<T>, dim3(nact), dim3(256), 0, sm, active, A, uniform, tab);
+}
+template void launch_class_rows<double>(hipStream_t, const int*, int, Coef7<double>, int*, double*);
+template void launch_class_rows<float>(hipStream_t, const int*, int, Coef7<float>, int*, float*);
 
 // P / S with NS red-black SOR sweeps of the block-local system (ghost values zero) from z = 0,
 // on the compact matrix above, in FP64: u = v / Ap; red cells first; each update
@@ -595,9 +645,9 @@ void launch_gsk(const BiOpts& o, hipStream_t sm, const int* active, int nact, co
 // LDS holds the operand's interior (NC values) and the ghost layers of the four side faces
 // (4 NF values, same layout as the halo); the two z ghosts of a column stay in registers.  In
 // FP64 that is 40 KiB, so four workgroups fit a CU.
-// REG 1 (FP32 bands, every block of the launch class-uniform): the bands come from the block's 27
-// class rows tab[slot][27][8] (the thread's column needs three: k = 0, inner, NB - 1), so no
-// per-cell band is read; REG 2 (mixed launch): so for the blocks with uni[slot] set.
+// REG 1 (every block of the launch class-uniform): the bands come from the block's 27 class rows
+// tab[slot][27][8] (the thread's column needs three: k = 0, inner, NB - 1), so no per-cell band is
+// read; REG 2 (mixed launch): so for the blocks with uni[slot] set.
 template <class T, int MODE, class TA = T, bool HR = false, bool CC = false, int REG = 0>
 __global__ __launch_bounds__(BI_NT) void bi_matvec_kernel(const int* __restrict__ active,
                                                           const DevBlock* __restrict__ blk,
@@ -605,7 +655,7 @@ __global__ __launch_bounds__(BI_NT) void bi_matvec_kernel(const int* __restrict_
                                                           Coef7<TA> A, BiVecs<T> V, double* __restrict__ part,
                                                           size_t nslots, const double* __restrict__ ce = nullptr,
                                                           double* __restrict__ bsy = nullptr,
-                                                          const float* __restrict__ tab = nullptr,
+                                                          const TA* __restrict__ tab = nullptr,
                                                           const int* __restrict__ uni = nullptr, int early = 0) {
   __shared__ T s[NC + 4 * NF];
   double* const red = reinterpret_cast<double*>(s);  // after the last read of s (block_sum syncs first)
@@ -639,9 +689,8 @@ __global__ __launch_bounds__(BI_NT) void bi_matvec_kernel(const int* __restrict_
     for (int f = 0; f < 4; f++) gv[f] = h[f * NF + t];
     zm = h[halo_index(4, tx, ty)];
     zp = h[halo_index(5, tx, ty)];
-    if (REG != 0 && cls) {
-      static_assert(REG == 0 || sizeof(TA) == 4, "class rows are FP32 bands");
-      const float* tr = tab + ((size_t)slot * 27 + stencil_class1(tx) + 3 * stencil_class1(ty)) * 8;
+    if (REG != 0) {  // rows exist for every block
+      const TA* tr = class_column(tab, slot, tx, ty);
 #pragma unroll
       for (int q = 0; q < 7; q++) {
         al[q] = tr[q];
@@ -658,63 +707,72 @@ __global__ __launch_bounds__(BI_NT) void bi_matvec_kernel(const int* __restrict_
   if (st[c].done) return;
   if (!early) stage_loads();
   const uint32_t local = (uint32_t)(slot - cs[c].slot_begin);
-  T a[KB][7], wv[KB];
-  auto load_batch = [&](int k0) {
+  // the rest in two forms, so that a class-uniform block's holds no per-cell bands
+  auto rest = [&](auto cls_tag) {
+    constexpr bool CLS = decltype(cls_tag)::value;
+    T a[KB][7], wv[KB];
+    auto load_batch = [&](int k0) {
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const int k = k0 + kk;
-      const size_t g = base + o0 + NF * k;
-      if (REG != 0 && cls) {
+      for (int kk = 0; kk < KB; kk++) {
+        const int k = k0 + kk;
+        const size_t g = base + o0 + NF * k;
+        if constexpr (!CLS) {
 #pragma unroll
-        for (int q = 0; q < 7; q++) a[kk][q] = (T)(k == 0 ? al[q] : k == NB - 1 ? ah[q] : ai[q]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 7; q++) a[kk][q] = (T)A.p[q][g];
+          for (int q = 0; q < 7; q++) a[kk][q] = (T)A.p[q][g];
+        }
+        wv[kk] = (MODE == 0 && HR) ? (T)shadow_value(local, (uint32_t)(g - base)) : w[g];
       }
-      wv[kk] = (MODE == 0 && HR) ? (T)shadow_value(local, (uint32_t)(g - base)) : w[g];
+    };
+    load_batch(0);  // in flight while the operand is staged
+    if constexpr (CC) {  // each thread corrects the values it stages
+      const DevBlock& Bk = blk[slot];
+      const double* e = ce + MODE * nslots;
+      const T eo = (T)e[slot];
+#pragma unroll
+      for (int k = 0; k < NB; k++) v[k] += eo;
+#pragma unroll
+      for (int f = 0; f < 4; f++) gv[f] += (T)e[ghost_source(Bk, slot, f, t & 15, t >> 4)];
+      zm += (T)e[ghost_source(Bk, slot, 4, tx, ty)];
+      zp += (T)e[ghost_source(Bk, slot, 5, tx, ty)];
+    }
+#pragma unroll
+    for (int k = 0; k < NB; k++) s[o0 + NF * k] = v[k];
+#pragma unroll
+    for (int f = 0; f < 4; f++) s[NC + f * NF + t] = gv[f];
+    __syncthreads();
+#pragma unroll
+    for (int k0 = 0; k0 < NB; k0 += KB) {
+      if (k0 > 0) load_batch(k0);
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++) {
+        const int k = k0 + kk;
+        const int li = o0 + NF * k;
+        const size_t g = base + li;
+        // a face lane reads the ghost layer (halo layout: face f at (a, b) = NC + f NF + a + NB b)
+        const T vxm = s[tx > 0 ? li - 1 : NC + halo_index(0, ty, k)];
+        const T vxp = s[tx < NB - 1 ? li + 1 : NC + halo_index(1, ty, k)];
+        const T vym = s[ty > 0 ? li - NB : NC + halo_index(2, tx, k)];
+        const T vyp = s[ty < NB - 1 ? li + NB : NC + halo_index(3, tx, k)];
+        const T vzm = k > 0 ? s[li - NF] : zm;
+        const T vzp = k < NB - 1 ? s[li + NF] : zp;
+        if constexpr (CLS) {
+#pragma unroll
+          for (int q = 0; q < 7; q++) a[kk][q] = k == 0 ? al[q] : k == NB - 1 ? ah[q] : ai[q];
+        }
+        // calc_ax order (bils.f90:195-202)
+        const T r = a[kk][1] * vxm + a[kk][2] * vxp + a[kk][3] * vym + a[kk][4] * vyp + a[kk][5] * vzm +
+                    a[kk][6] * vzp + a[kk][0] * s[li];
+        y[g] = r;
+        ys += (double)r;
+        d0 += (double)r * (double)wv[kk];
+        if (MODE == 1) d1 += (double)r * (double)r;
+      }
     }
   };
-  load_batch(0);  // in flight while the operand is staged
-  if constexpr (CC) {  // each thread corrects the values it stages
-    const DevBlock& Bk = blk[slot];
-    const double* e = ce + MODE * nslots;
-    const T eo = (T)e[slot];
-#pragma unroll
-    for (int k = 0; k < NB; k++) v[k] += eo;
-#pragma unroll
-    for (int f = 0; f < 4; f++) gv[f] += (T)e[ghost_source(Bk, slot, f, t & 15, t >> 4)];
-    zm += (T)e[ghost_source(Bk, slot, 4, tx, ty)];
-    zp += (T)e[ghost_source(Bk, slot, 5, tx, ty)];
-  }
-#pragma unroll
-  for (int k = 0; k < NB; k++) s[o0 + NF * k] = v[k];
-#pragma unroll
-  for (int f = 0; f < 4; f++) s[NC + f * NF + t] = gv[f];
-  __syncthreads();
-#pragma unroll
-  for (int k0 = 0; k0 < NB; k0 += KB) {
-    if (k0 > 0) load_batch(k0);
-#pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const int k = k0 + kk;
-      const int li = o0 + NF * k;
-      const size_t g = base + li;
-      // a face lane reads the ghost layer (halo layout: face f at (a, b) = NC + f NF + a + NB b)
-      const T vxm = s[tx > 0 ? li - 1 : NC + halo_index(0, ty, k)];
-      const T vxp = s[tx < NB - 1 ? li + 1 : NC + halo_index(1, ty, k)];
-      const T vym = s[ty > 0 ? li - NB : NC + halo_index(2, tx, k)];
-      const T vyp = s[ty < NB - 1 ? li + NB : NC + halo_index(3, tx, k)];
-      const T vzm = k > 0 ? s[li - NF] : zm;
-      const T vzp = k < NB - 1 ? s[li + NF] : zp;
-      // calc_ax order (bils.f90:195-202)
-      const T r = a[kk][1] * vxm + a[kk][2] * vxp + a[kk][3] * vym + a[kk][4] * vyp + a[kk][5] * vzm +
-                  a[kk][6] * vzp + a[kk][0] * s[li];
-      y[g] = r;
-      ys += (double)r;
-      d0 += (double)r * (double)wv[kk];
-      if (MODE == 1) d1 += (double)r * (double)r;
-    }
-  }
+  if (REG == 1 || (REG == 2 && cls))
+    rest(std::true_type{});
+  else if constexpr (REG != 1)
+    rest(std::false_type{});
   double s0 = block_sum<BI_NT>(d0, red);
   double s1 = MODE == 1 ? block_sum<BI_NT>(d1, red) : 0.0;
   if (t == 0) {
@@ -906,20 +964,20 @@ void launch_bicgstab_restart(hipStream_t sm, const int* active, int nact, const 
 template <class T>
 void launch_bicgstab_init(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                           SolveState* st, Coef7<T> A, const T* b, const T* x, const T* hx, BiVecs<T> V, double* part,
-                          size_t nslots, bool hash_r0, double* bsr) {
+                          size_t nslots, bool hash_r0, double* bsr, ClassRows<T> R) {
   if (!nact) return;
   if (hash_r0)
     hipLaunchKernelGGL((bi_init_kernel<T, true>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs, st, A, b, x, hx, V,
-                       part, nslots, bsr);
+                       part, nslots, bsr, R);
   else
     hipLaunchKernelGGL((bi_init_kernel<T, false>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs, st, A, b, x, hx,
-                       V, part, nslots, bsr);
+                       V, part, nslots, bsr, R);
 }
 
 template <class T>
 void launch_bicgstab_iter(hipStream_t sm, const int* active, int nact, const int* caseact, int ncase,
                           const DevBlock* blk, const DevCase* cs, SolveState* st, Coef7<T> A, T* x, BiVecs<T> V,
-                          double* part, size_t nslots, int count, int mask, const BiOpts& o) {
+                          double* part, size_t nslots, int count, int mask, const BiOpts& o, ClassRows<T> R) {
   // mask bits 0-4 select P, Q, S, T, XR; bit 5 leaves out the per-case finalisations; bit 8
   // splits the coarse corrections of the two-level methods into stages of their own (bits 6, 7).
   // Multiplicative two-level methods (count > 0): bit 9 has this iteration's first coarse
@@ -958,10 +1016,10 @@ void launch_bicgstab_iter(hipStream_t sm, const int* active, int nact, const int
                          *o.M64, Vd, count);
     else if (dbl && o.A32)
       hipLaunchKernelGGL((bi_precond_kernel<double, MODE, float>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs,
-                         st, *o.A32, Vd, count);
+                         st, *o.A32, Vd, count, ClassRows<float>());
     else
       hipLaunchKernelGGL((bi_precond_kernel<T, MODE>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs, st, A, V,
-                         count);
+                         count, R);
   };
   // the T stage keeps its partials in part[2..3] (XR reads them while writing part[0..1])
   auto matvec = [&](auto mode_tag) {
@@ -1007,8 +1065,11 @@ void launch_bicgstab_iter(hipStream_t sm, const int* active, int nact, const int
     else if (dbl && o.A32)
       hipLaunchKernelGGL((bi_matvec_kernel<double, MODE, float>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs,
                          st, *o.A32, Vd, part, nslots, nullptr, nullptr, nullptr, nullptr, early);
+    else if (R.uni)
+      hipLaunchKernelGGL((bi_matvec_kernel<T, MODE, T, false, false, 2>), dim3(nact), dim3(BI_NT), 0, sm, active, blk,
+                         cs, st, A, V, part, nslots, nullptr, nullptr, R.tab, R.uni, early);
     else
-      hipLaunchKernelGGL((bi_matvec_kernel<T, MODE>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs, st, A, V,
+      hipLaunchKernelGGL((bi_matvec_kernel<T, MODE, T>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs, st, A, V,
                          part, nslots, nullptr, nullptr, nullptr, nullptr, early);
   };
   using M0 = std::integral_constant<int, 0>;
@@ -1065,10 +1126,10 @@ void launch_bicgstab_iter(hipStream_t sm, const int* active, int nact, const int
 #define INST(T)                                                                                                     \
   template void launch_bicgstab_init<T>(hipStream_t, const int*, int, const DevBlock*, const DevCase*, SolveState*,  \
                                         Coef7<T>, const T*, const T*, const T*, BiVecs<T>, double*, size_t, bool,    \
-                                        double*);                                                                    \
+                                        double*, ClassRows<T>);                                                                    \
   template void launch_bicgstab_iter<T>(hipStream_t, const int*, int, const int*, int, const DevBlock*,            \
                                         const DevCase*, SolveState*, Coef7<T>, T*, BiVecs<T>, double*, size_t, int,  \
-                                        int, const BiOpts&);                                                         \
+                                        int, const BiOpts&, ClassRows<T>);                                                         \
   template void launch_bicgstab_reanchor<T>(hipStream_t, const int*, int, const DevBlock*, const SolveState*,         \
                                             BiVecs<T>, double*, size_t);                                             \
   template void launch_bicgstab_restart<T>(hipStream_t, const int*, int, const DevBlock*, const SolveState*, BiVecs<T>); \

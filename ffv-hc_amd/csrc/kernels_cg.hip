@@ -26,7 +26,7 @@ __global__ __launch_bounds__(CG_NT) void cg_init_kernel(const int* __restrict__ 
                                                         const DevCase* __restrict__ cs, SolveState* __restrict__ st,
                                                         Coef7<T> A, const T* __restrict__ bv, const T* __restrict__ x,
                                                         const T* __restrict__ hx, T* __restrict__ r,
-                                                        double* __restrict__ part, size_t nslots) {
+                                                        double* __restrict__ part, size_t nslots, ClassRows<T> R) {
   __shared__ T s[LP * LP * LP];
   __shared__ double red[CG_NT / 64];
   const int slot = active[blockIdx.x];
@@ -38,33 +38,36 @@ __global__ __launch_bounds__(CG_NT) void cg_init_kernel(const int* __restrict__ 
   const T omega = (T)st[c].omega;
   constexpr int KB = Batch<T>::K;
   double bb = 0.0, rz = 0.0;
+  by_class(R, slot, [&](auto cls) {
+    const ColumnBands<T, decltype(cls)::value> W(R, slot, tx, ty);
 #pragma unroll
-  for (int k0 = 0; k0 < NB; k0 += KB) {
-    T a[KB][7], b0[KB];
+    for (int k0 = 0; k0 < NB; k0 += KB) {
+      T a[KB][7], b0[KB];
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
 #pragma unroll
-      for (int q = 0; q < 7; q++) a[kk][q] = A.p[q][g];
-      b0[kk] = bv[g];
+        for (int q = 0; q < 7; q++) a[kk][q] = W(A, q, k0 + kk, g);
+        b0[kk] = bv[g];
+      }
+      if (k0 == 0) {
+        stage_block<T, CG_NT>(s, x, hx, slot);
+        __syncthreads();
+      }
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        const int li = lds(tx, ty, k0 + kk);
+        const T rr = b0[kk] - a[kk][1] * s[li - 1] - a[kk][2] * s[li + 1] - a[kk][3] * s[li - LP] -
+                     a[kk][4] * s[li + LP] - a[kk][5] * s[li - LP * LP] - a[kk][6] * s[li + LP * LP] -
+                     a[kk][0] * s[li];
+        r[g] = rr;
+        const T z = jacobi_z<T>(rr, a[kk][0], omega);
+        bb += (double)b0[kk] * (double)b0[kk];
+        rz += (double)rr * (double)z;
+      }
     }
-    if (k0 == 0) {
-      stage_block<T, CG_NT>(s, x, hx, slot);
-      __syncthreads();
-    }
-#pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      const int li = lds(tx, ty, k0 + kk);
-      const T rr = b0[kk] - a[kk][1] * s[li - 1] - a[kk][2] * s[li + 1] - a[kk][3] * s[li - LP] -
-                   a[kk][4] * s[li + LP] - a[kk][5] * s[li - LP * LP] - a[kk][6] * s[li + LP * LP] -
-                   a[kk][0] * s[li];
-      r[g] = rr;
-      const T z = jacobi_z<T>(rr, a[kk][0], omega);
-      bb += (double)b0[kk] * (double)b0[kk];
-      rz += (double)rr * (double)z;
-    }
-  }
+  });
   double sb = block_sum<CG_NT>(bb, red);
   double sz = block_sum<CG_NT>(rz, red);
   if (t == 0) {
@@ -77,7 +80,7 @@ template <class T>
 __global__ __launch_bounds__(CG_NT) void cg_p_kernel(const int* __restrict__ active, const DevBlock* __restrict__ blk,
                                                      const DevCase* __restrict__ cs, const SolveState* __restrict__ st,
                                                      Coef7<T> A, const T* __restrict__ r, T* __restrict__ p,
-                                                     T* __restrict__ hp, int count, int bcg) {
+                                                     T* __restrict__ hp, int count, int bcg, ClassRows<T> R) {
   __shared__ T s[LP * LP * LP];
   const int slot = active[blockIdx.x];
   const DevBlock& B = blk[slot];
@@ -88,25 +91,30 @@ __global__ __launch_bounds__(CG_NT) void cg_p_kernel(const int* __restrict__ act
   const T omega = (T)st[c].omega;
   const T beta = (T)st[c].beta;
   constexpr int KB = Batch<T>::K;
+  by_class(R, slot, [&](auto cls) {
+    constexpr bool CLS = decltype(cls)::value;
+    const T* tr = CLS ? class_column(R.tab, slot, tx, ty) : nullptr;
+    const T alo = CLS ? tr[0] : (T)0, ain = CLS ? tr[9 * 8] : (T)0, ahi = CLS ? tr[18 * 8] : (T)0;
 #pragma unroll
-  for (int k0 = 0; k0 < NB; k0 += KB) {
-    T rv[KB], ap[KB], pv[KB];
+    for (int k0 = 0; k0 < NB; k0 += KB) {
+      T rv[KB], ap[KB], pv[KB];
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      rv[kk] = r[g];
-      ap[kk] = A.p[0][g];
-      if (count != 1) pv[kk] = p[g];
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        rv[kk] = r[g];
+        ap[kk] = CLS ? (k0 + kk == 0 ? alo : k0 + kk == NB - 1 ? ahi : ain) : A.p[0][g];
+        if (count != 1) pv[kk] = p[g];
+      }
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        const T z = jacobi_z<T>(rv[kk], ap[kk], omega);
+        const T pn = (count == 1) ? z : z + beta * pv[kk];
+        p[g] = pn;
+        s[lds(tx, ty, k0 + kk)] = pn;
+      }
     }
-#pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      const T z = jacobi_z<T>(rv[kk], ap[kk], omega);
-      const T pn = (count == 1) ? z : z + beta * pv[kk];
-      p[g] = pn;
-      s[lds(tx, ty, k0 + kk)] = pn;
-    }
-  }
+  });
   __syncthreads();
   push_halo<T, CG_NT>(B, cs[c], bcg, slot, [&](int i, int j, int k) { return s[lds(i, j, k)]; }, hp, hp);
 }
@@ -115,7 +123,7 @@ template <class T>
 __global__ __launch_bounds__(CG_NT) void cg_q_kernel(const int* __restrict__ active, const DevBlock* __restrict__ blk,
                                                      const DevCase* __restrict__ cs, SolveState* __restrict__ st,
                                                      Coef7<T> A, const T* __restrict__ p, const T* __restrict__ hp,
-                                                     T* __restrict__ q, double* __restrict__ part) {
+                                                     T* __restrict__ q, double* __restrict__ part, ClassRows<T> R) {
   __shared__ T s[LP * LP * LP];
   __shared__ double red[CG_NT / 64];
   const int slot = active[blockIdx.x];
@@ -126,30 +134,33 @@ __global__ __launch_bounds__(CG_NT) void cg_q_kernel(const int* __restrict__ act
   const size_t base = (size_t)slot * NC;
   constexpr int KB = Batch<T>::K;
   double qp = 0.0;
+  by_class(R, slot, [&](auto cls) {
+    const ColumnBands<T, decltype(cls)::value> W(R, slot, tx, ty);
 #pragma unroll
-  for (int k0 = 0; k0 < NB; k0 += KB) {
-    T a[KB][7];
+    for (int k0 = 0; k0 < NB; k0 += KB) {
+      T a[KB][7];
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
 #pragma unroll
-      for (int w = 0; w < 7; w++) a[kk][w] = A.p[w][g];
+        for (int w = 0; w < 7; w++) a[kk][w] = W(A, w, k0 + kk, g);
+      }
+      if (k0 == 0) {
+        stage_block<T, CG_NT>(s, p, hp, slot);
+        __syncthreads();
+      }
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        const int li = lds(tx, ty, k0 + kk);
+        const T pv = s[li];
+        const T qv = a[kk][1] * s[li - 1] + a[kk][2] * s[li + 1] + a[kk][3] * s[li - LP] + a[kk][4] * s[li + LP] +
+                     a[kk][5] * s[li - LP * LP] + a[kk][6] * s[li + LP * LP] + a[kk][0] * pv;
+        q[g] = qv;
+        qp += (double)qv * (double)pv;
+      }
     }
-    if (k0 == 0) {
-      stage_block<T, CG_NT>(s, p, hp, slot);
-      __syncthreads();
-    }
-#pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      const int li = lds(tx, ty, k0 + kk);
-      const T pv = s[li];
-      const T qv = a[kk][1] * s[li - 1] + a[kk][2] * s[li + 1] + a[kk][3] * s[li - LP] + a[kk][4] * s[li + LP] +
-                   a[kk][5] * s[li - LP * LP] + a[kk][6] * s[li + LP * LP] + a[kk][0] * pv;
-      q[g] = qv;
-      qp += (double)qv * (double)pv;
-    }
-  }
+  });
   double sq = block_sum<CG_NT>(qp, red);
   if (t == 0) part[slot] = sq;
 }
@@ -159,7 +170,8 @@ __global__ __launch_bounds__(CG_NT) void cg_xr_kernel(const int* __restrict__ ac
                                                       const DevCase* __restrict__ cs, SolveState* __restrict__ st,
                                                       Coef7<T> A, T* __restrict__ x, T* __restrict__ r,
                                                       const T* __restrict__ p, const T* __restrict__ q,
-                                                      double* __restrict__ part, size_t nslots, int count) {
+                                                      double* __restrict__ part, size_t nslots, int count,
+                                                      ClassRows<T> R) {
   __shared__ double red[CG_NT / 64];
   const int slot = active[blockIdx.x];
   const DevBlock& B = blk[slot];
@@ -172,29 +184,34 @@ __global__ __launch_bounds__(CG_NT) void cg_xr_kernel(const int* __restrict__ ac
   const T omega = (T)st[c].omega;
   constexpr int KB = Batch<T>::K;
   double rr = 0.0, rz = 0.0;
+  by_class(R, slot, [&](auto cls) {
+    constexpr bool CLS = decltype(cls)::value;
+    const T* tr = CLS ? class_column(R.tab, slot, tx, ty) : nullptr;
+    const T alo = CLS ? tr[0] : (T)0, ain = CLS ? tr[9 * 8] : (T)0, ahi = CLS ? tr[18 * 8] : (T)0;
 #pragma unroll
-  for (int k0 = 0; k0 < NB; k0 += KB) {
-    T xv[KB], pv[KB], rv[KB], qv[KB], ap[KB];
+    for (int k0 = 0; k0 < NB; k0 += KB) {
+      T xv[KB], pv[KB], rv[KB], qv[KB], ap[KB];
 #pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      xv[kk] = x[g];
-      pv[kk] = p[g];
-      rv[kk] = r[g];
-      qv[kk] = q[g];
-      ap[kk] = A.p[0][g];
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        xv[kk] = x[g];
+        pv[kk] = p[g];
+        rv[kk] = r[g];
+        qv[kk] = q[g];
+        ap[kk] = CLS ? (k0 + kk == 0 ? alo : k0 + kk == NB - 1 ? ahi : ain) : A.p[0][g];
+      }
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++) {
+        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+        x[g] = xv[kk] + alpha * pv[kk];
+        const T rn = rv[kk] + nalpha * qv[kk];
+        r[g] = rn;
+        const T z = jacobi_z<T>(rn, ap[kk], omega);
+        rr += (double)rn * (double)rn;
+        rz += (double)rn * (double)z;
+      }
     }
-#pragma unroll
-    for (int kk = 0; kk < KB; kk++) {
-      const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-      x[g] = xv[kk] + alpha * pv[kk];
-      const T rn = rv[kk] + nalpha * qv[kk];
-      r[g] = rn;
-      const T z = jacobi_z<T>(rn, ap[kk], omega);
-      rr += (double)rn * (double)rn;
-      rz += (double)rn * (double)z;
-    }
-  }
+  });
   double sr = block_sum<CG_NT>(rr, red);
   double sz = block_sum<CG_NT>(rz, red);
   if (t == 0) {
@@ -205,37 +222,42 @@ __global__ __launch_bounds__(CG_NT) void cg_xr_kernel(const int* __restrict__ ac
 
 template <class T>
 void launch_cg_init(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs, SolveState* st,
-                    Coef7<T> A, const T* b, const T* x, const T* hx, T* r, double* part, size_t nslots) {
+                    Coef7<T> A, const T* b, const T* x, const T* hx, T* r, double* part, size_t nslots,
+                    ClassRows<T> R) {
   if (nact) hipLaunchKernelGGL(cg_init_kernel<T>, dim3(nact), dim3(CG_NT), 0, sm, active, blk, cs, st, A, b, x, hx, r,
-                               part, nslots);
+                               part, nslots, R);
 }
 template <class T>
 void launch_cg_p(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
-                 const SolveState* st, Coef7<T> A, const T* r, T* p, T* hp, int count, int bcg) {
+                 const SolveState* st, Coef7<T> A, const T* r, T* p, T* hp, int count, int bcg,
+                 ClassRows<T> R) {
   if (nact) hipLaunchKernelGGL(cg_p_kernel<T>, dim3(nact), dim3(CG_NT), 0, sm, active, blk, cs, st, A, r, p, hp,
-                               count, bcg);
+                               count, bcg, R);
 }
 template <class T>
 void launch_cg_q(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs, SolveState* st,
-                 Coef7<T> A, const T* p, const T* hp, T* q, double* part) {
-  if (nact) hipLaunchKernelGGL(cg_q_kernel<T>, dim3(nact), dim3(CG_NT), 0, sm, active, blk, cs, st, A, p, hp, q, part);
+                 Coef7<T> A, const T* p, const T* hp, T* q, double* part,
+                 ClassRows<T> R) {
+  if (nact) hipLaunchKernelGGL(cg_q_kernel<T>, dim3(nact), dim3(CG_NT), 0, sm, active, blk, cs, st, A, p, hp, q, part,
+                               R);
 }
 template <class T>
 void launch_cg_xr(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs, SolveState* st,
-                  Coef7<T> A, T* x, T* r, const T* p, const T* q, double* part, size_t nslots, int count) {
+                  Coef7<T> A, T* x, T* r, const T* p, const T* q, double* part, size_t nslots, int count,
+                  ClassRows<T> R) {
   if (nact) hipLaunchKernelGGL(cg_xr_kernel<T>, dim3(nact), dim3(CG_NT), 0, sm, active, blk, cs, st, A, x, r, p, q,
-                               part, nslots, count);
+                               part, nslots, count, R);
 }
 
 #define INST(T)                                                                                                   \
   template void launch_cg_init<T>(hipStream_t, const int*, int, const DevBlock*, const DevCase*, SolveState*,      \
-                                  Coef7<T>, const T*, const T*, const T*, T*, double*, size_t);                   \
+                                  Coef7<T>, const T*, const T*, const T*, T*, double*, size_t, ClassRows<T>);     \
   template void launch_cg_p<T>(hipStream_t, const int*, int, const DevBlock*, const DevCase*, const SolveState*,   \
-                               Coef7<T>, const T*, T*, T*, int, int);                                              \
+                               Coef7<T>, const T*, T*, T*, int, int, ClassRows<T>);                                \
   template void launch_cg_q<T>(hipStream_t, const int*, int, const DevBlock*, const DevCase*, SolveState*,         \
-                               Coef7<T>, const T*, const T*, T*, double*);                                         \
+                               Coef7<T>, const T*, const T*, T*, double*, ClassRows<T>);                           \
   template void launch_cg_xr<T>(hipStream_t, const int*, int, const DevBlock*, const DevCase*, SolveState*,        \
-                                Coef7<T>, T*, T*, const T*, const T*, double*, size_t, int);
+                                Coef7<T>, T*, T*, const T*, const T*, double*, size_t, int, ClassRows<T>);
 INST(double)
 INST(float)
 #undef INST

@@ -84,18 +84,24 @@ __global__ __launch_bounds__(256) void ghost_pull_kernel(const int* __restrict__
 // ------------------------------------------------------------------------------------------
 constexpr int RB_NT = 512;
 
+// Bound by memory.  Where the block is class-uniform (R) the bands come from two class rows a thread
+// instead of 56 B a cell: 30 B/cell move instead of 86.  Every load of the half column is issued
+// before the first LDS store.  Four wavefronts a SIMD (two workgroups a CU) is what 128 registers
+// allow; a non-uniform block reads the black cells' bands twice, from the cache, to stay below that.
+// 1,128 blocks FP64: 105.6 us (3.7 TB/s) with per-cell bands, 37 us (3.7 TB/s on a third of the
+// bytes) with class rows.
 // MODE 0: FFVILS::RBGS iteration.  MODE 1: FFVILS::Jacobi iteration (jacobi_smoother,
 // bils.f90:5-55: every cell from the old values, then the ghost fill).  MODE 2: the sweep of
 // FFVILS::RBGS_WithFixedAverage (FFVILS.h:596-659): x^n unshifted, no ghost push, and the block
 // sum of x^n (sf3d_calc_sum) into part[2][slot]; shift_push_kernel then removes the mean.
 template <class T, int MODE>
-__global__ __launch_bounds__(RB_NT) void rbgs_iter_kernel(const int* __restrict__ active, const DevBlock* __restrict__ blk,
+__global__ __launch_bounds__(RB_NT, 4) void rbgs_iter_kernel(const int* __restrict__ active, const DevBlock* __restrict__ blk,
                                                           const DevCase* __restrict__ cs, SolveState* __restrict__ st,
                                                           Coef7<T> A,
                                                           const T* __restrict__ bv, const T* __restrict__ xin,
                                                           T* __restrict__ xout, const T* __restrict__ hin,
                                                           T* __restrict__ hout, double* __restrict__ part,
-                                                          size_t nslots, int n, int bcg) {
+                                                          size_t nslots, int n, int bcg, ClassRows<T> R) {
   __shared__ T s[LP * LP * LP];
   __shared__ double red[RB_NT / 64];
   const int slot = active[blockIdx.x];
@@ -106,84 +112,118 @@ __global__ __launch_bounds__(RB_NT) void rbgs_iter_kernel(const int* __restrict_
   const int tx = t & 15, ty = (t >> 4) & 15, tz = t >> 8;
   const size_t base = (size_t)slot * NC;
   const size_t hbase = (size_t)slot * NH;
-#pragma unroll
-  for (int kk = 0; kk < 8; kk++) {
-    const int k = tz * 8 + kk;
-    s[lds(tx, ty, k)] = xin[base + tx + NB * (ty + NB * k)];
-  }
-  for (int q = t; q < NH; q += RB_NT) {
-    int f = q >> 8, p = q & 255, i, j, k;
-    face_cell(f, p & 15, p >> 4, -1, i, j, k);
-    s[lds(i, j, k)] = hin[hbase + q];
-  }
-  __syncthreads();
+  const size_t g0 = base + tx + NB * (ty + NB * (tz * 8));  // this thread's half column
   const bool sweep = n <= st[c].countMax;
   const T omega = (T)st[c].omega;
   const int par = (tx + ty) & 1;
-  double rr = 0.0, bb = 0.0;
-  T xr[4], sA[4][7], sb[4], xj[8];
+  double rr = 0.0, bb = 0.0, xsum = 0.0;
+  by_class(R, slot, [&](auto cls) {
+    constexpr bool CLS = decltype(cls)::value;
+    // CLS: the class rows of the half column's end cell (k = 0 below, NB - 1 above) and of the others
+    T in[7], end[7];
+    if constexpr (CLS) {
+      const T* tr = class_column(R.tab, slot, tx, ty);
 #pragma unroll
-  for (int m = 0; m < 4; m++) {
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int k = tz * 8 + 2 * m + h;
-      const bool isred = (h == par);
-      const size_t g = base + tx + NB * (ty + NB * k);
-      const int li = lds(tx, ty, k);
-      T a[7];
-#pragma unroll
-      for (int q = 0; q < 7; q++) a[q] = A.p[q][g];
-      const T b0 = bv[g];
-      const T xp = s[li];
-      const T rs = b0 - a[1] * s[li - 1] - a[2] * s[li + 1] - a[3] * s[li - LP] - a[4] * s[li + LP] -
-                   a[5] * s[li - LP * LP] - a[6] * s[li + LP * LP];
-      const T r = rs - a[0] * xp;
-      rr += (double)r * (double)r;
-      if (n == 1) bb += (double)b0 * (double)b0;
-      if (MODE == 1) {
-        xj[2 * m + h] = xp - omega * (xp - rs / a[0]);
-      } else if (isred) {
-        xr[m] = xp - omega * (xp - rs / a[0]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 7; q++) sA[m][q] = a[q];
-        sb[m] = b0;
+      for (int q = 0; q < 7; q++) {
+        in[q] = tr[9 * 8 + q];
+        end[q] = tr[(tz ? 18 * 8 : 0) + q];
       }
     }
-  }
-  double xsum = 0.0;
-  if (sweep && MODE == 1) {
-    __syncthreads();
+    T xv[8], hv[NH / RB_NT], b0[8];
 #pragma unroll
-    for (int q = 0; q < 8; q++) s[lds(tx, ty, tz * 8 + q)] = xj[q];
-    __syncthreads();
+    for (int kk = 0; kk < 8; kk++) xv[kk] = xin[g0 + NF * kk];
 #pragma unroll
-    for (int q = 0; q < 8; q++) xout[base + tx + NB * (ty + NB * (tz * 8 + q))] = xj[q];
-    push_halo<T, RB_NT>(B, cs[c], bcg, slot, [&](int i, int j, int k) { return s[lds(i, j, k)]; }, hin, hout);
-  } else if (sweep) {
-    __syncthreads();
+    for (int q = 0; q < NH / RB_NT; q++) hv[q] = hin[hbase + t + q * RB_NT];
 #pragma unroll
-    for (int m = 0; m < 4; m++) s[lds(tx, ty, tz * 8 + 2 * m + par)] = xr[m];
+    for (int kk = 0; kk < 8; kk++) b0[kk] = bv[g0 + NF * kk];
+#pragma unroll
+    for (int kk = 0; kk < 8; kk++) s[lds(tx, ty, tz * 8 + kk)] = xv[kk];
+#pragma unroll
+    for (int q = 0; q < NH / RB_NT; q++) {
+      const int w = t + q * RB_NT, f = w >> 8, p = w & 255;
+      int i, j, k;
+      face_cell(f, p & 15, p >> 4, -1, i, j, k);
+      s[lds(i, j, k)] = hv[q];
+    }
     __syncthreads();
+    // b less the six neighbour products of cell kk with the coefficients a
+    auto off_sum = [&](int kk, T bk, const T* a) -> T {
+      const int li = lds(tx, ty, tz * 8 + kk);
+      return bk - a[1] * s[li - 1] - a[2] * s[li + 1] - a[3] * s[li - LP] - a[4] * s[li + LP] -
+             a[5] * s[li - LP * LP] - a[6] * s[li + LP * LP];
+    };
+    // the residual of every cell, the new value of the red ones (MODE 1: of all); per pair of cells
+    // (2m, 2m + 1) one is red, chosen by the column's parity, so the division is done once
+    T xj[8], sb[4], sx[4];
+    // coefficients of cell kk (a constant once unrolled)
+    auto coef = [&](int kk, T* a) {
+#pragma unroll
+      for (int q = 0; q < 7; q++) {
+        if constexpr (CLS)
+          a[q] = kk == 0 ? (tz ? in[q] : end[q]) : kk == 7 ? (tz ? end[q] : in[q]) : in[q];
+        else
+          a[q] = A.p[q][g0 + NF * kk];
+      }
+    };
 #pragma unroll
     for (int m = 0; m < 4; m++) {
-      const int k = tz * 8 + 2 * m + (1 - par);
-      const int li = lds(tx, ty, k);
-      const T xp = s[li];
-      const T rs = sb[m] - sA[m][1] * s[li - 1] - sA[m][2] * s[li + 1] - sA[m][3] * s[li - LP] -
-                   sA[m][4] * s[li + LP] - sA[m][5] * s[li - LP * LP] - sA[m][6] * s[li + LP * LP];
-      s[li] = xp - omega * (xp - rs / sA[m][0]);
-    }
-    __syncthreads();
+      T a[2][7], rs[2];
 #pragma unroll
-    for (int kk = 0; kk < 8; kk++) {
-      const int k = tz * 8 + kk;
-      const T v = s[lds(tx, ty, k)];
-      xout[base + tx + NB * (ty + NB * k)] = v;
-      if (MODE == 2) xsum += (double)v;
+      for (int h = 0; h < 2; h++) {
+        const int kk = 2 * m + h;
+        coef(kk, a[h]);
+        rs[h] = off_sum(kk, b0[kk], a[h]);
+        const T r = rs[h] - a[h][0] * xv[kk];
+        rr += (double)r * (double)r;
+        if (n == 1) bb += (double)b0[kk] * (double)b0[kk];
+        if (MODE == 1) xj[kk] = xv[kk] - omega * (xv[kk] - rs[h] / a[h][0]);
+      }
+      if (MODE != 1) {
+        const T xp = par ? xv[2 * m + 1] : xv[2 * m];
+        xj[m] = xp - omega * (xp - (par ? rs[1] : rs[0]) / (par ? a[1][0] : a[0][0]));
+        sx[m] = par ? xv[2 * m] : xv[2 * m + 1];
+        sb[m] = par ? b0[2 * m] : b0[2 * m + 1];
+      }
     }
-    if (MODE == 0)
-      push_halo<T, RB_NT>(B, cs[c], bcg, slot, [&](int i, int j, int k) { return s[lds(i, j, k)]; }, hin, hout);
+    if (!sweep) return;
+    __syncthreads();
+    if (MODE == 1) {
+#pragma unroll
+      for (int kk = 0; kk < 8; kk++) {
+        s[lds(tx, ty, tz * 8 + kk)] = xj[kk];
+        xout[g0 + NF * kk] = xj[kk];
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < 4; m++) s[lds(tx, ty, tz * 8 + 2 * m + par)] = xj[m];
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        const int kk = 2 * m + 1 - par;
+        T a[7];
+        if constexpr (CLS) {
+          const bool e = m == 0 ? (par && !tz) : m == 3 ? (!par && tz) : false;
+#pragma unroll
+          for (int q = 0; q < 7; q++) a[q] = e ? end[q] : in[q];
+        } else {  // read again (from the cache): holding them would cost 56 registers
+#pragma unroll
+          for (int q = 0; q < 7; q++) a[q] = A.p[q][g0 + NF * kk];
+        }
+        const T xb = sx[m] - omega * (sx[m] - off_sum(kk, sb[m], a) / a[0]);
+        s[lds(tx, ty, tz * 8 + kk)] = xb;
+        const T x0 = par ? xb : xj[m], x1 = par ? xj[m] : xb;  // cells 2m and 2m + 1
+        xout[g0 + NF * (2 * m)] = x0;
+        xout[g0 + NF * (2 * m + 1)] = x1;
+        if (MODE == 2) {
+          xsum += (double)x0;
+          xsum += (double)x1;
+        }
+      }
+    }
+  });
+  if (sweep && MODE != 2) {
+    __syncthreads();
+    push_halo<T, RB_NT>(B, cs[c], bcg, slot, [&](int i, int j, int k) { return s[lds(i, j, k)]; }, hin, hout);
   }
   // residual of x^{n-1} (and b.b on the first launch)
   double rsum = block_sum<RB_NT>(rr, red);
@@ -266,17 +306,17 @@ void launch_ghost_pull(hipStream_t sm, const int* active, int nact, const DevBlo
 template <class T>
 void launch_rbgs_iter(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                       SolveState* st, Coef7<T> A, const T* b, const T* xin, T* xout, const T* hin,
-                      T* hout, double* part, size_t nslots, int n, int bcg, int mode) {
+                      T* hout, double* part, size_t nslots, int n, int bcg, int mode, ClassRows<T> R) {
   if (nact == 0) return;
   if (mode == 0)
     hipLaunchKernelGGL((rbgs_iter_kernel<T, 0>), dim3(nact), dim3(RB_NT), 0, sm, active, blk, cs, st, A, b, xin,
-                       xout, hin, hout, part, nslots, n, bcg);
+                       xout, hin, hout, part, nslots, n, bcg, R);
   else if (mode == 1)
     hipLaunchKernelGGL((rbgs_iter_kernel<T, 1>), dim3(nact), dim3(RB_NT), 0, sm, active, blk, cs, st, A, b, xin,
-                       xout, hin, hout, part, nslots, n, bcg);
+                       xout, hin, hout, part, nslots, n, bcg, R);
   else
     hipLaunchKernelGGL((rbgs_iter_kernel<T, 2>), dim3(nact), dim3(RB_NT), 0, sm, active, blk, cs, st, A, b, xin,
-                       xout, hin, hout, part, nslots, n, bcg);
+                       xout, hin, hout, part, nslots, n, bcg, R);
 }
 
 template <class T>
@@ -315,10 +355,10 @@ template void launch_ghost_pull<float>(hipStream_t, const int*, int, const DevBl
                                        float*, int, int, bool);
 template void launch_rbgs_iter<double>(hipStream_t, const int*, int, const DevBlock*, const DevCase*, SolveState*,
                                        Coef7<double>, const double*, const double*, double*, const double*, double*,
-                                       double*, size_t, int, int, int);
+                                       double*, size_t, int, int, int, ClassRows<double>);
 template void launch_rbgs_iter<float>(hipStream_t, const int*, int, const DevBlock*, const DevCase*, SolveState*,
                                       Coef7<float>, const float*, const float*, float*, const float*, float*, double*,
-                                      size_t, int, int, int);
+                                      size_t, int, int, int, ClassRows<float>);
 template void launch_shift_push<double>(hipStream_t, const int*, int, const DevBlock*, const DevCase*,
                                         const SolveState*, double*, const double*, double*, int);
 template void launch_shift_push<float>(hipStream_t, const int*, int, const DevBlock*, const DevCase*,

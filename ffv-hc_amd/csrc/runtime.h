@@ -151,6 +151,10 @@ struct ffvhc_ctx {
   float* dctab = nullptr;
   void* dctrec = nullptr;
   bool classes = true;
+  // class rows of the reference solvers' matrix (FP64 or FP32, made at the start of each solve; apart
+  // from the tables above, which the time step keeps): per slot the flag and 27 rows of 8
+  int* drows_uni = nullptr;
+  void* drows = nullptr;
   // shadow residual of the compact-record methods: r0 = r (default, the reference's choice) or the
   // seeded hash vector (FFVHC_OPTION_SHADOW 1: on the 1,128-block Poisson benchmark 2-4 fewer iterations for methods 24-27 and no
   // r0 reads, on the flow past a sphere 15% more iterations a step)

@@ -101,8 +101,9 @@ long long ffvhc_ctx_device_bytes(const ffvhc_ctx* ctx);
 /* FFVHC_OPTION_CLASSES: 1 (default) lets the compact-record methods (ffvhc_solve_mixed 11-28)
  * find the blocks whose seven bands are the same within each of the 27 stencil position classes
  * (face layers, edges, corners, inside: every block without cut cells) and read those blocks'
- * bands and preconditioner records from 27 rows instead of per cell; 0 reads every block per
- * cell.  The results are identical. */
+ * bands and preconditioner records from 27 rows instead of per cell, and the FP64 / FP32
+ * solvers of the reference (RBGS, Jacobi, CG, BiCGSTAB) read such a block's bands from 27 rows of
+ * the matrix's own precision; 0 reads every block per cell.  The results are identical. */
 #define FFVHC_OPTION_CLASSES 2
 /* FFVHC_OPTION_SHADOW: 0 (default) the compact-record methods (11-28) take the reference's shadow
  * residual r0 = r; 1 the seeded hash vector of method 10, computed where it is read (no r0
