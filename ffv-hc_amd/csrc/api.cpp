@@ -329,6 +329,9 @@ void ffvhc_ctx_destroy(ffvhc_ctx* c) {
   (void)hipFree(c->dctrec);
   (void)hipFree(c->drows_uni);
   (void)hipFree(c->drows);
+  (void)hipFree(c->drows_ex);
+  (void)hipFree(c->dcex);
+  (void)hipFree(c->dwords);
   (void)hipFree(c->dcut);
   (void)hipFree(c->dflag);
   (void)hipFree(c->dcid);

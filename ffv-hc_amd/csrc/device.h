@@ -98,12 +98,14 @@ struct Coef7 {
 };
 
 // Class rows of a 7-point matrix: uni[slot] = 1 when every cell of the block has bitwise the bands of
-// its position class, tab[slot][27][8] the 27 rows (the eighth entry unused); uni null: none were
-// made and every block reads its per-cell bands.
+// its position class, tab[slot][27][8] the 27 rows (the eighth entry unused), ex[slot][512] the cells
+// that differ from their row (one byte per half column, bit k & 7); uni null: none were made and
+// every block reads its per-cell bands.
 template <class T>
 struct ClassRows {
   const int* uni = nullptr;
   const T* tab = nullptr;
+  const unsigned char* ex = nullptr;
 };
 
 // BiCGSTAB work vectors r r0 p p_ q_ s s_ t_ and the ghost layers of p_ and s_

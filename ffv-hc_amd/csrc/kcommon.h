@@ -139,6 +139,10 @@ struct ColumnBands {
   }
 };
 
+// halves of a packed pair of FP16 couplings (the preconditioner records of kernels_bicg.hip)
+__device__ inline double half_lo(uint32_t u) { return (double)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xffffu)); }
+__device__ inline double half_hi(uint32_t u) { return (double)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16)); }
+
 // f(true_type) for a class-uniform block, f(false_type) else (uniform over the workgroup)
 template <class T, class F>
 __device__ inline void by_class(const ClassRows<T>& R, int slot, const F& f) {
@@ -163,6 +167,22 @@ __device__ inline void converged(SolveState& s, double rr, int count) {
   } else if (count >= s.countMax) {
     s.done = 1;
     s.count = s.countMax + 1;  // loop exhausted: for(count=1; count<=countMax; ++count)
+  }
+}
+
+// The end of a PCG iteration (FFVILS.h:759-787): t0 = r.r (IsConverged), t1 = the next r.z
+__device__ inline void cg_end(SolveState& S, double t0, double t1, int n) {
+  S.iter = n;
+  converged(S, t0, n);
+  if (S.done) return;
+  S.rr0 = S.rr1;
+  if (fabs(t1) < FLT_MIN) {
+    S.residual = t1;
+    S.count = 0;
+    S.done = 1;
+  } else {
+    S.rr1 = t1;
+    S.beta = t1 / S.rr0;
   }
 }
 
@@ -254,6 +274,30 @@ __device__ inline void fin_bi_xr_store(SolveState& S, const FinXr& f, int n, dou
 }
 
 
+__device__ inline int coarse_pitch(int n) { return (n + 3) & ~3; }
+
+// e = A_c^-1 c for each active block's row: one wavefront per row, the row read as float4
+// (pitch coarse_pitch(n), offsets off[case]); c(b) gives the coarse right-hand side of block b
+// (0 past n); the sum order is fixed (lane-strided float4 groups, then the wave reduction), so a
+// case's result does not depend on what else is batched with it
+template <class Rhs>
+__device__ inline double coarse_row_dot(const float* __restrict__ row, int n, int lane, const Rhs& c) {
+  const float4* r4 = reinterpret_cast<const float4*>(row);
+  double s = 0.0;
+  const int nq = coarse_pitch(n) / 4;
+#pragma unroll 4
+  for (int q = lane; q < nq; q += 64) {
+    const float4 v = r4[q];
+    const int b = 4 * q;
+    s += (double)v.x * c(b);
+    s += (double)v.y * c(b + 1);
+    s += (double)v.z * c(b + 2);
+    s += (double)v.w * c(b + 3);
+  }
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  return s;
+}
+
 // Neighbour slot a face position (a, b) of face f takes its ghost value from.
 __device__ inline int ghost_source(const DevBlock& B, int slot, int f, int a, int b) {
   switch (B.ftype[f]) {
@@ -270,13 +314,22 @@ __device__ inline int ghost_source(const DevBlock& B, int slot, int f, int a, in
   }
 }
 
+// How push_halo stores a ghost value: a plain store, or (in a kernel whose workgroups read one
+// another's ghosts while it runs) one that is visible to the whole device once it completes.
+struct PutPlain {
+  template <class T>
+  __device__ void operator()(T* p, T v) const {
+    *p = v;
+  }
+};
+
 // Push this block's ghost-layer contributions into the next halo buffer: its own outer faces
 // (bcx.f90), the facing layer of same-level neighbours, F2C means into a coarser neighbour's
 // quarter face and C2F trilinear values into each finer neighbour (Scalar3DUpdater1 semantics).
 // `L(i,j,k)` reads the block's new interior (LDS).
-template <class T, int NT, class Acc>
+template <class T, int NT, class Acc, class Put = PutPlain>
 __device__ inline void push_halo(const DevBlock& B, const DevCase& C, int bcg, int slot, const Acc& L,
-                                 const T* __restrict__ hin, T* __restrict__ hout) {
+                                 const T* __restrict__ hin, T* __restrict__ hout, const Put& put = Put()) {
   const int t = threadIdx.x;
   const size_t hbase = (size_t)slot * NH;
   for (int f = 0; f < 6; f++) {
@@ -292,14 +345,14 @@ __device__ inline void push_halo(const DevBlock& B, const DevCase& C, int bcg, i
         T xa = L(i, j, k);
         face_cell(f ^ 1, a, b, 0, i, j, k);
         T xf = L(i, j, k);
-        hout[hbase + f * NF + p] = outer_value<T>(f, type, xc, xa, xf, hin[hbase + f * NF + p], pp);
+        put(&hout[hbase + f * NF + p], outer_value<T>(f, type, xc, xa, xf, hin[hbase + f * NF + p], pp));
       }
     } else if (ft == FACE_SAME) {
       const size_t nb = (size_t)B.nbr[f][0] * NH + (f ^ 1) * NF;
       for (int p = t; p < NF; p += NT) {
         int i, j, k;
         face_cell(f, p & 15, p >> 4, 0, i, j, k);
-        hout[nb + p] = L(i, j, k);
+        put(&hout[nb + p], (T)L(i, j, k));
       }
     } else if (ft == FACE_COARSER) {
       const size_t cb = (size_t)B.nbr[f][0] * NH;
@@ -307,13 +360,13 @@ __device__ inline void push_halo(const DevBlock& B, const DevCase& C, int bcg, i
       sub_origins_ab(f, B.sub[f], oa, ob);
       for (int p = t; p < NF / 4; p += NT) {
         int ca = (p & 7) + 8 * oa, cbb = (p >> 3) + 8 * ob;
-        hout[cb + halo_index(f ^ 1, ca, cbb)] = f2c_mean<T>(f ^ 1, ca, cbb, L, false);
+        put(&hout[cb + halo_index(f ^ 1, ca, cbb)], f2c_mean<T>(f ^ 1, ca, cbb, L, false));
       }
     } else {
       for (int q = t; q < 4 * NF; q += NT) {
         const int sub = q >> 8, p = q & 255;
         const size_t fb = (size_t)B.nbr[f][sub] * NH;
-        hout[fb + halo_index(f ^ 1, p & 15, p >> 4)] = c2f_trilinear<T>(f ^ 1, sub, p & 15, p >> 4, L);
+        put(&hout[fb + halo_index(f ^ 1, p & 15, p >> 4)], c2f_trilinear<T>(f ^ 1, sub, p & 15, p >> 4, L));
       }
     }
   }

@@ -96,6 +96,7 @@ struct BiOpts {
   const float* tab = nullptr;
   const uint4* trec = nullptr;
   const int* uni = nullptr;
+  const unsigned char* ex = nullptr;  // the cells that differ from their class row (launch_stencil_classes)
   int nreg = 0, nirr = 0;
 };
 
@@ -113,6 +114,69 @@ void launch_bicgstab_shadow(hipStream_t sm, const int* active, int nact, const D
 template <class T>
 void launch_bicgstab_restart(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const SolveState* st,
                              BiVecs<T> V);
+// Resident solvers (kernels_resident.hip): one launch runs up to `turns` iterations of a solve whose
+// blocks (one workgroup each, at most RS_MAX) are on the chip together.
+constexpr int RS_MAX = 256;
+constexpr int RS_COPIES = 8;                // copies of a block's words in a meeting
+constexpr int RS_WORDS = 9 * RS_COPIES + 1;  // 8-byte words per slot
+
+struct ResidentBicg {
+  const int* active;
+  const DevBlock* blk;
+  const DevCase* cs;
+  SolveState* st;
+  Coef7<double> A64;      // Jacobi: the matrix and its class rows
+  ClassRows<double> R64;
+  Coef7<float> A32;       // two-level: the FP32 matrix, its class rows, the preconditioner records ...
+  ClassRows<float> R32;
+  const uint4* rec;
+  const uint4* trec;
+  int sweeps;
+  const float* cinv;      // ... and the coarse inverses and block sums (BiOpts)
+  const long long* coff;
+  double* ce;
+  double* x;
+  BiVecs<double> V;
+  unsigned long long* words;  // RS_WORDS per slot, unset before each launch
+  size_t nslots;
+  int turns;
+};
+template <class T>
+struct ResidentCg {
+  const int* active;
+  const DevBlock* blk;
+  const DevCase* cs;
+  SolveState* st;
+  Coef7<T> A;
+  ClassRows<T> R;
+  T *x, *r, *p, *hp;
+  unsigned long long* words;
+  size_t nslots;
+  int turns;
+};
+template <class T>
+struct ResidentRelax {
+  const int* active;
+  const DevBlock* blk;
+  const DevCase* cs;
+  SolveState* st;
+  Coef7<T> A;
+  ClassRows<T> R;
+  const T* b;
+  T* x;
+  T* h[2];
+  int bcg;
+  unsigned long long* words;
+  size_t nslots;
+  int turns;
+};
+template <class T>
+bool launch_resident_cg(hipStream_t sm, int nact, int* limit, ResidentCg<T>& args);
+template <class T>
+bool launch_resident_relax(hipStream_t sm, int nact, int mode, int* limit, ResidentRelax<T>& args);
+// limit: how many workgroups of this kernel the device holds (-1: not asked yet); false: not launched
+bool launch_resident_bicg(hipStream_t sm, int nact, bool two, int* limit, ResidentBicg& args);
+void launch_unset_words(hipStream_t sm, const int* active, int nact, unsigned long long* words, size_t nslots);
 void launch_defect(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                    SolveState* st, Coef7<double> A, const double* b, const double* x, const double* hx, float* r32,
                    double* part, size_t nslots, int outer);
@@ -121,13 +185,15 @@ void launch_add_correction(hipStream_t sm, const int* active, int nact, const De
 void launch_convert(hipStream_t sm, const int* active, int nact, float* y, const double* x);
 // Compact GS preconditioner records (16 bytes per cell: 1 / Ap in FP32, A_q / Ap in FP16)
 void launch_gs_pack(hipStream_t sm, const int* active, int nact, Coef7<double> A, uint4* rec);
-// Stencil position classes of each block (uniform[slot] = 1 when the block is class-uniform) and
-// its 27 class rows: FP32 bands tab[slot][27][8] and preconditioner records trec[slot][27]
+// Stencil position classes of each block (uniform[slot] = 1 when the block is class-uniform), its
+// 27 class rows (FP32 bands tab[slot][27][8] and preconditioner records trec[slot][27]) and the cells
+// that differ from their row, ex[slot][512] (one byte per half column, bit k & 7)
 void launch_stencil_classes(hipStream_t sm, const int* active, int nact, Coef7<double> A, int* uniform, float* tab,
-                            uint4* trec);
-// the flags and the 27 rows in the matrix's own precision (the reference solvers)
+                            unsigned char* ex, uint4* trec);
+// the same with rows in the matrix's own precision (the reference solvers)
 template <class T>
-void launch_class_rows(hipStream_t sm, const int* active, int nact, Coef7<T> A, int* uniform, T* tab);
+void launch_class_rows(hipStream_t sm, const int* active, int nact, Coef7<T> A, int* uniform, T* tab,
+                       unsigned char* ex);
 // coarse operator rows (25 doubles per slot), dense Gauss-Jordan inversion, FP32 copy, apply
 void launch_coarse_rows(hipStream_t sm, const int* active, int nact, const DevBlock* blk, Coef7<double> A,
                         double* rows);

@@ -274,9 +274,6 @@ __device__ inline uint32_t half_bits(double v) {
   const _Float16 h = (_Float16)(v > lim ? lim : v < -lim ? -lim : v);
   return (uint32_t)__builtin_bit_cast(uint16_t, h);
 }
-__device__ inline double half_lo(uint32_t u) { return (double)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xffffu)); }
-__device__ inline double half_hi(uint32_t u) { return (double)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16)); }
-
 __device__ inline uint4 gs_record(const Coef7<double>& A, size_t g) {
   const double d = A.p[0][g];
   const double inv = d != 0.0 ? 1.0 / d : 0.0;  // a zero pivot decouples the cell in M
@@ -303,82 +300,97 @@ void launch_gs_pack(hipStream_t sm, const int* active, int nact, Coef7<double> A
 // and level interfaces (those change the coefficients of a whole face layer alike).  For such a
 // block the 27 rows -- as FP32 bands (8 floats each, the eighth unused) and as preconditioner
 // records -- stand for the per-cell arrays, bit for bit.
-__global__ __launch_bounds__(256) void stencil_class_kernel(const int* __restrict__ active, Coef7<double> A,
-                                                            int* __restrict__ uniform, float* __restrict__ tab,
-                                                            uint4* __restrict__ trec) {
+// Two candidates a class (its lowest- and its highest-index cell); the row is the one more cells
+// agree with, which matters to blocks that a body cuts only: ex[slot][512] then marks the cells that
+// differ from their row, one byte per half column (i, j, k >= 8 or not), bit = k & 7.  Bound by the one
+// pass over the seven bands: a column's 16 planes of a band are loaded at once and compared bitwise,
+// no load waits on a comparison (2,480 blocks FP64: 150 us, 3.8 TB/s).
+__device__ inline int stencil_last1(int c) { return c == 0 ? 0 : c == 2 ? NB - 1 : NB - 2; }
+
+template <class T, class TR, bool REC>
+__global__ __launch_bounds__(256, 4) void class_rows_kernel(const int* __restrict__ active, Coef7<T> A,
+                                                         int* __restrict__ uniform, TR* __restrict__ tab,
+                                                         unsigned char* __restrict__ ex, uint4* __restrict__ trec) {
+  using Bits = std::conditional_t<sizeof(T) == 8, unsigned long long, unsigned int>;
+  __shared__ T rep[2][27 * 8];
+  __shared__ int differ[2][27];
   const int slot = active[blockIdx.x];
   const size_t base = (size_t)slot * NC;
   const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
-  const int rx = stencil_rep1(stencil_class1(tx)), ry = stencil_rep1(stencil_class1(ty));
-  bool same = true;
-  for (int k = 0; k < NB; k++) {
-    const size_t g = base + tx + NB * (ty + NB * k);
-    const size_t r = base + rx + NB * (ry + NB * stencil_rep1(stencil_class1(k)));
+  // cell of candidate w of class row
+  auto cell = [](int w, int row) {
+    const int c0 = row % 3, c1 = (row / 3) % 3, c2 = row / 9;
+    return w ? stencil_last1(c0) + NB * (stencil_last1(c1) + NB * stencil_last1(c2))
+             : stencil_rep1(c0) + NB * (stencil_rep1(c1) + NB * stencil_rep1(c2));
+  };
+  if (t < 27 * 8)
+    for (int w = 0; w < 2; w++) {
+      const size_t g = base + cell(w, t >> 3);
+      T v = 0;
 #pragma unroll
-    for (int q = 0; q < 7; q++)
-      same = same && __double_as_longlong(A.p[q][g]) == __double_as_longlong(A.p[q][r]);
-  }
-  const int all = __syncthreads_and(same ? 1 : 0);
-  if (t < 27) {
-    const size_t r = base + stencil_rep1(t % 3) + NB * (stencil_rep1((t / 3) % 3) + NB * stencil_rep1(t / 9));
-    float* row = tab + ((size_t)slot * 27 + t) * 8;
+      for (int b = 0; b < 7; b++)
+        if (b == (t & 7)) v = A.p[b][g];
+      rep[w][t] = v;
+    }
+  if (t < 54) differ[t / 27][t % 27] = 0;
+  __syncthreads();
+  const int row0 = stencil_class1(tx) + 3 * stencil_class1(ty);  // k = 0; the others are 9 and 18 on
+  unsigned m0 = 0, m1 = 0;  // planes of the column that differ from candidate 0, 1
+  T v[2][NB];
+  auto load = [&](int q) {
+    const T* const b = A.p[q] + base + tx + NB * ty;
 #pragma unroll
-    for (int q = 0; q < 7; q++) row[q] = (float)A.p[q][r];
-    row[7] = 0.0f;
-    trec[(size_t)slot * 27 + t] = gs_record(A, r);
+    for (int k = 0; k < NB; k++) v[q & 1][k] = b[NF * k];
+  };
+  load(0);
+#pragma unroll
+  for (int q = 0; q < 7; q++) {
+    if (q < 6) load(q + 1);
+    __builtin_amdgcn_sched_barrier(0);  // one band ahead, not all seven: registers
+#pragma unroll
+    for (int k = 0; k < NB; k++) {
+      const int i = (row0 + 9 * stencil_class1(k)) * 8 + q;
+      m0 |= (unsigned)(__builtin_bit_cast(Bits, v[q & 1][k]) != __builtin_bit_cast(Bits, rep[0][i])) << k;
+      m1 |= (unsigned)(__builtin_bit_cast(Bits, v[q & 1][k]) != __builtin_bit_cast(Bits, rep[1][i])) << k;
+    }
+    asm volatile("" : "+v"(m0), "+v"(m1));  // the bits are gathered band by band (not 224 comparisons later)
   }
+  const unsigned part[3] = {1u, 0x7ffeu, 0x8000u};  // the planes of the column's three classes
+#pragma unroll
+  for (int z = 0; z < 3; z++) {
+    if (m0 & part[z]) atomicAdd(&differ[0][row0 + 9 * z], __popc(m0 & part[z]));
+    if (m1 & part[z]) atomicAdd(&differ[1][row0 + 9 * z], __popc(m1 & part[z]));
+  }
+  __syncthreads();
+  unsigned m = 0;
+#pragma unroll
+  for (int z = 0; z < 3; z++) m |= (differ[1][row0 + 9 * z] < differ[0][row0 + 9 * z] ? m1 : m0) & part[z];
+  ex[(size_t)slot * 512 + t] = (unsigned char)(m & 0xffu);
+  ex[(size_t)slot * 512 + 256 + t] = (unsigned char)(m >> 8);
+  if (t < 27 * 8) tab[(size_t)slot * 27 * 8 + t] = (TR)rep[differ[1][t >> 3] < differ[0][t >> 3]][t];
+  if constexpr (REC)
+    if (t < 27) trec[(size_t)slot * 27 + t] = gs_record(A, base + cell(differ[1][t] < differ[0][t], t));
+  const int all = __syncthreads_and(m == 0 ? 1 : 0);
   if (t == 0) uniform[slot] = all;
 }
 
 void launch_stencil_classes(hipStream_t sm, const int* active, int nact, Coef7<double> A, int* uniform, float* tab,
-                            uint4* trec) {
-  if (nact) hipLaunchKernelGGL(stencil_class_kernel, dim3(nact), dim3(256), 0, sm, active, A, uniform, tab, trec);
+                            unsigned char* ex, uint4* trec) {
+  if (nact)
+    hipLaunchKernelGGL((class_rows_kernel<double, float, true>), dim3(nact), dim3(256), 0, sm, active, A, uniform, tab,
+                       ex, trec);
 }
 
-// The same flags and the 27 rows in the matrix's own precision, for the reference solvers (no FP32
-// copy, no records).  Bound by the one pass over the seven bands: the representative rows wait in
-// LDS and the difference is gathered bitwise, so no load waits on a comparison.
+// The same in the matrix's own precision, for the reference solvers (no FP32 copy, no records)
 template <class T>
-__global__ __launch_bounds__(256) void class_rows_kernel(const int* __restrict__ active, Coef7<T> A,
-                                                         int* __restrict__ uniform, T* __restrict__ tab) {
-  using Bits = std::conditional_t<sizeof(T) == 8, unsigned long long, unsigned int>;
-  __shared__ T rep[27 * 8];
-  const int slot = active[blockIdx.x];
-  const size_t base = (size_t)slot * NC;
-  const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
-  if (t < 27 * 8) {
-    const int row = t >> 3, q = t & 7;
-    const size_t r = base + stencil_rep1(row % 3) + NB * (stencil_rep1((row / 3) % 3) + NB * stencil_rep1(row / 9));
-    T v = 0;
-#pragma unroll
-    for (int b = 0; b < 7; b++)
-      if (b == q) v = A.p[b][r];
-    rep[t] = v;
-    tab[(size_t)slot * 27 * 8 + t] = v;
-  }
-  __syncthreads();
-  const T* const mine = rep + (stencil_class1(tx) + 3 * stencil_class1(ty)) * 8;
-  Bits diff = 0;
-#pragma unroll
-  for (int q = 0; q < 7; q++) {
-    const T* const b = A.p[q] + base + tx + NB * ty;
-    T v[NB];
-#pragma unroll
-    for (int k = 0; k < NB; k++) v[k] = b[NF * k];
-#pragma unroll
-    for (int k = 0; k < NB; k++)
-      diff |= __builtin_bit_cast(Bits, v[k]) ^ __builtin_bit_cast(Bits, mine[stencil_class1(k) * 9 * 8 + q]);
-  }
-  const int all = __syncthreads_and(diff == 0 ? 1 : 0);
-  if (t == 0) uniform[slot] = all;
+void launch_class_rows(hipStream_t sm, const int* active, int nact, Coef7<T> A, int* uniform, T* tab,
+                       unsigned char* ex) {
+  if (nact)
+    hipLaunchKernelGGL((class_rows_kernel<T, T, false>), dim3(nact), dim3(256), 0, sm, active, A, uniform, tab, ex,
+                       nullptr);
 }
-
-template <class T>
-void launch_class_rows(hipStream_t sm, const int* active, int nact, Coef7<T> A, int* uniform, T* tab) {
-  if (nact) hipLaunchKernelGGL(class_rows_kernel<T>, dim3(nact), dim3(256), 0, sm, active, A, uniform, tab);
-}
-template void launch_class_rows<double>(hipStream_t, const int*, int, Coef7<double>, int*, double*);
-template void launch_class_rows<float>(hipStream_t, const int*, int, Coef7<float>, int*, float*);
+template void launch_class_rows<double>(hipStream_t, const int*, int, Coef7<double>, int*, double*, unsigned char*);
+template void launch_class_rows<float>(hipStream_t, const int*, int, Coef7<float>, int*, float*, unsigned char*);
 
 // P / S with NS red-black SOR sweeps of the block-local system (ghost values zero) from z = 0,
 // on the compact matrix above, in FP64: u = v / Ap; red cells first; each update

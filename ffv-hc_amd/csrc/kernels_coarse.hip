@@ -295,30 +295,6 @@ void launch_to_f32(hipStream_t sm, const double* x, float* y, int n, int np) {
   if (total) hipLaunchKernelGGL(to_f32_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, sm, x, y, n, np);
 }
 
-__device__ inline int coarse_pitch(int n) { return (n + 3) & ~3; }
-
-// e = A_c^-1 c for each active block's row: one wavefront per row, the row read as float4
-// (pitch coarse_pitch(n), offsets off[case]); c(b) gives the coarse right-hand side of block b
-// (0 past n); the sum order is fixed (lane-strided float4 groups, then the wave reduction), so a
-// case's result does not depend on what else is batched with it
-template <class Rhs>
-__device__ inline double coarse_row_dot(const float* __restrict__ row, int n, int lane, const Rhs& c) {
-  const float4* r4 = reinterpret_cast<const float4*>(row);
-  double s = 0.0;
-  const int nq = coarse_pitch(n) / 4;
-#pragma unroll 4
-  for (int q = lane; q < nq; q += 64) {
-    const float4 v = r4[q];
-    const int b = 4 * q;
-    s += (double)v.x * c(b);
-    s += (double)v.y * c(b + 1);
-    s += (double)v.z * c(b + 2);
-    s += (double)v.w * c(b + 3);
-  }
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  return s;
-}
-
 // The same sum with the row's first CA_PRE float4 per lane already loaded (pre[i] = r4[lane + 64 i])
 constexpr int CA_PRE = 6;
 template <class Rhs>

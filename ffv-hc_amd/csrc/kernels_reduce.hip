@@ -82,20 +82,8 @@ __global__ __launch_bounds__(FIN_NT) void finalize_kernel(const int* __restrict_
     case FIN_CG_ALPHA:  // FFVILS.h:745-749: alpha = rr1 / (q.p)
       S.alpha = S.rr1 / t0;
       break;
-    case FIN_CG_XR:  // FFVILS.h:759-787: t0 = r.r (IsConverged), t1 = next r.z
-      S.iter = arg;
-      converged(S, t0, arg);
-      if (!S.done) {
-        S.rr0 = S.rr1;
-        if (fabs(t1) < FLT_MIN) {
-          S.residual = t1;
-          S.count = 0;
-          S.done = 1;
-        } else {
-          S.rr1 = t1;
-          S.beta = t1 / S.rr0;
-        }
-      }
+    case FIN_CG_XR:  // FFVILS.h:759-787
+      cg_end(S, t0, t1, arg);
       break;
     case FIN_RBGS:  // launch arg = n computed ||b - A x^{n-1}||^2 (and b.b when n == 1)
       S.iter = arg;

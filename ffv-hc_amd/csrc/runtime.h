@@ -148,13 +148,20 @@ struct ffvhc_ctx {
   // stencil classes of the compact-record methods (FFVHC_OPTION_CLASSES): per slot the
   // class-uniform flag and the 27 class rows as FP32 bands and as 16-byte preconditioner records
   int* dcuni = nullptr;
+  unsigned char* dcex = nullptr;  // cells that differ from their class row
   float* dctab = nullptr;
   void* dctrec = nullptr;
   bool classes = true;
   // class rows of the reference solvers' matrix (FP64 or FP32, made at the start of each solve; apart
   // from the tables above, which the time step keeps): per slot the flag and 27 rows of 8
   int* drows_uni = nullptr;
+  unsigned char* drows_ex = nullptr;
   void* drows = nullptr;
+  // resident solvers: their words (RS_WORDS per slot), how many workgroups of each kernel the device holds
+  // (-1: not asked yet), and whether they are used (off after a wait in one ended without everyone)
+  unsigned long long* dwords = nullptr;
+  int resident_limit[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
+  bool resident = true;
   // shadow residual of the compact-record methods: r0 = r (default, the reference's choice) or the
   // seeded hash vector (FFVHC_OPTION_SHADOW 1: on the 1,128-block Poisson benchmark 2-4 fewer iterations for methods 24-27 and no
   // r0 reads, on the flow past a sphere 15% more iterations a step)

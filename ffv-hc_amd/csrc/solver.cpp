@@ -85,13 +85,62 @@ int class_rows(ffvhc_ctx* c, const Coef7<T>& K, int turns, ClassRows<T>* R) {
   const size_t cap = (size_t)c->cap;
   if (!c->drows) {
     HIPCHK(hipMalloc(&c->drows_uni, cap * sizeof(int)));
+    HIPCHK(hipMalloc(&c->drows_ex, cap * 512));
     HIPCHK(hipMalloc(&c->drows, cap * 27 * 8 * sizeof(double)));
   }
-  launch_class_rows<T>(c->sm, c->dactive, c->nactive, K, c->drows_uni, (T*)c->drows);
+  launch_class_rows<T>(c->sm, c->dactive, c->nactive, K, c->drows_uni, (T*)c->drows,
+                       c->drows_ex);
   HIPCHK(hipGetLastError());
   R->uni = c->drows_uni;
   R->tab = (const T*)c->drows;
+  R->ex = c->drows_ex;
   return 0;
+}
+
+// Iterations a resident solver runs in one launch: bounds how long a launch holds the device (a few
+// tens of milliseconds); a solve that needs more continues in the next launch.
+constexpr int kResidentTurns = 2048;
+
+enum Resident { NOT_RESIDENT, RESIDENT_DONE, RESIDENT_FAILED };
+enum { RL_BICG = 0, RL_CG = 2, RL_RELAX = 4 };  // kernels in ffvhc_ctx::resident_limit
+
+// Whether the resident kernels (kernels_resident.hip) may run the active blocks, their words made.  The
+// line lies at one block per compute unit: below it resident solves were faster at every size tried, from
+// 1 to 256 blocks (two-level BiCGSTAB 1.4-1.6x, Jacobi BiCGSTAB 1.8-2.2x, PCG 2.4-3.6x, RBGS and
+// Jacobi 1.3-1.8x against one launch per stage); above it the blocks' vectors no longer fit on the chip.
+bool resident_ready(ffvhc_ctx* c) {
+  if (!c->resident || c->nactive < 1 || c->nactive > RS_MAX) return false;
+  if (!c->dwords &&
+      hipMalloc(&c->dwords, sizeof(unsigned long long) * RS_WORDS * (size_t)c->cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return true;
+}
+
+// Launches a resident kernel (go: false when it does not fit the device or is refused) until the solve
+// has ended.  NOT_RESIDENT: nothing was launched.  RESIDENT_FAILED: a wait ended without everyone; the
+// context then solves with one launch per stage.
+template <class Go>
+Resident resident_run(ffvhc_ctx* c, SolveState* st, std::vector<SolveState>& hst, const std::vector<int>& ids,
+                      const Go& go, int* rc) {
+  bool done = false, any = false;
+  while (!done) {
+    launch_unset_words(c->sm, c->dactive, c->nactive, c->dwords, (size_t)c->cap);
+    bool failed = !go();
+    if (failed && !any) return NOT_RESIDENT;
+    any = true;
+    if (!failed) {
+      *rc = read_state(c, st, hst, ids, &done);
+      if (*rc) return RESIDENT_DONE;
+      for (int id : ids) failed = failed || hst[id].parity < 0;
+    }
+    if (failed) {
+      c->resident = false;
+      return RESIDENT_FAILED;
+    }
+  }
+  return RESIDENT_DONE;
 }
 
 // RBGS (mode 0), Jacobi (mode 1) or RBGS with fixed average (mode 2) on field x (ping-pong),
@@ -111,6 +160,35 @@ int rbgs_core(ffvhc_ctx* c, int xf, Coef7<T> K, const T* bv, int bcg, double ome
   T* hs[2] = {(T*)X.h[0], (T*)X.h[1]};
   int n = 1, batch = kBatchMin;
   bool done = false;
+  if (mode < 2 && R.uni && resident_ready(c)) {
+    ResidentRelax<T> a{};
+    a.active = c->dactive;
+    a.blk = c->dblk;
+    a.cs = c->dcase;
+    a.st = st;
+    a.A = K;
+    a.R = R;
+    a.b = bv;
+    a.x = xs[0];
+    a.h[0] = hs[0];
+    a.h[1] = hs[1];
+    a.bcg = bcg;
+    a.words = c->dwords;
+    a.nslots = (size_t)c->cap;
+    a.turns = kResidentTurns;
+    int* limit = &c->resident_limit[RL_RELAX + 2 * mode + (sizeof(T) == 4)];
+    int rc = 0;
+    const Resident where = resident_run(
+        c, st, hst, ids, [&] { return launch_resident_relax<T>(c->sm, c->nactive, mode, limit, a); }, &rc);
+    if (rc) return rc;
+    // both halo buffers are written by then: the sweeps cannot be run again from x
+    if (where == RESIDENT_FAILED) return fail(-2, "resident solve: the device did not run its workgroups together");
+    if (where == RESIDENT_DONE) {
+      if (launched)
+        for (int id : ids) *launched = std::max(*launched, hst[id].iter);
+      return 0;
+    }
+  }
   while (!done) {
     int last = std::min(n + batch - 1, countMax + 1);
     for (; n <= last; n++)
@@ -156,6 +234,29 @@ int cg_core(ffvhc_ctx* c, int xf, Coef7<T> K, const T* bv, int bcg, double omega
   fin(c, st, FIN_CG_INIT, 0);
   int n = 1, batch = kBatchMin;
   bool done = false;
+  if (R.uni && resident_ready(c)) {
+    ResidentCg<T> a{};
+    a.active = c->dactive;
+    a.blk = c->dblk;
+    a.cs = c->dcase;
+    a.st = st;
+    a.A = K;
+    a.R = R;
+    a.x = (T*)X.d[0];
+    a.r = (T*)Rf.d[0];
+    a.p = (T*)Pf.d[0];
+    a.hp = (T*)Pf.h[0];
+    a.words = c->dwords;
+    a.nslots = (size_t)c->cap;
+    a.turns = kResidentTurns;
+    const Resident where = resident_run(
+        c, st, hst, ids,
+        [&] { return launch_resident_cg<T>(c->sm, c->nactive, &c->resident_limit[RL_CG + (sizeof(T) == 4)], a); }, &rc);
+    if (rc) return rc;
+    if (where == RESIDENT_FAILED)  // again from the x there is (a starting guess like any other)
+      return cg_core<T>(c, xf, K, bv, bcg, omega, countMax, eps, st, hst, outer, launched);
+    done = where == RESIDENT_DONE;
+  }
   while (!done) {
     int last = std::min(n + batch - 1, countMax);
     for (; n <= last; n++) {
@@ -196,6 +297,50 @@ int bicg_vectors(ffvhc_ctx* c, BiVecs<T>* V) {
   V->hpp = (T*)c->fields[f[3]].h[0];
   V->hss = (T*)c->fields[f[6]].h[0];
   return 0;
+}
+
+// Runs the iterations of a BiCGSTAB whose initialisation is done in the resident kernel; not for the
+// forms that kernel does not have (FP32 vectors, the one-level and additive preconditioners, the
+// seeded shadow residual, graph replay, no class rows).
+template <class T>
+Resident bicgstab_resident(ffvhc_ctx* c, T* x, const Coef7<T>& K, const BiVecs<T>& V, SolveState* st,
+                           std::vector<SolveState>& hst, const std::vector<int>& ids, const BiOpts& o,
+                           const ClassRows<T>& R, int* rc) {
+  if constexpr (sizeof(T) == 4) {
+    return NOT_RESIDENT;
+  } else {
+    const bool two = o.gs == BiOpts::GSC && o.cinv && o.mult && !o.hash_r0 && o.trec;
+    const bool jacobi = o.gs == BiOpts::NONE && !o.A32 && R.uni;
+    if (c->graphs || !(two || jacobi) || !resident_ready(c)) return NOT_RESIDENT;
+    ResidentBicg a{};
+    a.active = c->dactive;
+    a.blk = c->dblk;
+    a.cs = c->dcase;
+    a.st = st;
+    if (two) {
+      a.A32 = *o.A32;
+      a.R32.uni = o.uni;
+      a.R32.tab = o.tab;
+      a.R32.ex = o.ex;
+      a.rec = o.rec;
+      a.trec = o.trec;
+      a.sweeps = o.sweeps;
+      a.cinv = o.cinv;
+      a.coff = o.coff;
+      a.ce = o.ce;
+    } else {
+      a.A64 = K;
+      a.R64 = R;
+    }
+    a.x = x;
+    a.V = V;
+    a.words = c->dwords;
+    a.nslots = (size_t)c->cap;
+    a.turns = kResidentTurns;
+    return resident_run(
+        c, st, hst, ids,
+        [&] { return launch_resident_bicg(c->sm, c->nactive, two, &c->resident_limit[RL_BICG + two], a); }, rc);
+  }
 }
 
 template <class T>
@@ -247,6 +392,12 @@ int bicgstab_core(ffvhc_ctx* c, int xf, Coef7<T> K, const T* bv, int bcg, double
   // next iteration's first coarse application; the batch's last iteration has its own launch, so
   // the state the host reads after the batch is complete
   const bool fuse = c->fuse_fin && !exec && opts.gs == BiOpts::GSC && opts.cinv && opts.mult;
+  int rcr = 0;
+  const Resident where = bicgstab_resident<T>(c, (T*)X.d[0], K, V, st, hst, ids, opts, R, &rcr);
+  if (rcr) return rcr;
+  if (where == RESIDENT_FAILED)  // again from the x there is (a starting guess like any other)
+    return bicgstab_core<T>(c, xf, K, bv, bcg, omega, countMax, eps, st, hst, outer, launched, opts);
+  done = where == RESIDENT_DONE;
   while (!done) {
     int last = std::min(n + batch - 1, countMax);
     const int first = n;
@@ -674,10 +825,12 @@ int class_launch(ffvhc_ctx* c, const Coef7<double>& K) {
   const size_t cap = (size_t)c->cap;
   if (!c->dcuni) {
     HIPCHK(hipMalloc(&c->dcuni, cap * sizeof(int)));
+    HIPCHK(hipMalloc(&c->dcex, cap * 512));
     HIPCHK(hipMalloc(&c->dctab, cap * 27 * 8 * sizeof(float)));
     HIPCHK(hipMalloc(&c->dctrec, cap * 27 * sizeof(uint4)));
   }
-  launch_stencil_classes(c->sm, c->dactive, c->nactive, K, c->dcuni, c->dctab, (uint4*)c->dctrec);
+  launch_stencil_classes(c->sm, c->dactive, c->nactive, K, c->dcuni, c->dctab, c->dcex,
+                         (uint4*)c->dctrec);
   HIPCHK(hipGetLastError());
   c->hcuni.resize(cap);
   HIPCHK(hipMemcpyAsync(c->hcuni.data(), c->dcuni, cap * sizeof(int), hipMemcpyDeviceToHost, c->sm));
@@ -690,6 +843,7 @@ void class_finish(ffvhc_ctx* c, BiOpts* o) {
   o->tab = c->dctab;
   o->trec = (const uint4*)c->dctrec;
   o->uni = c->dcuni;
+  o->ex = c->dcex;
   o->nreg = nreg;
   o->nirr = c->nactive - nreg;
 }
@@ -1184,6 +1338,10 @@ int ffvhc_ctx_set_option(ffvhc_ctx* c, int option, int value) {
   }
   if (option == FFVHC_OPTION_FUSE_FIN) {
     c->fuse_fin = value != 0;
+    return 0;
+  }
+  if (option == FFVHC_OPTION_RESIDENT) {
+    c->resident = value != 0;
     return 0;
   }
   if (option == FFVHC_OPTION_COARSE_GEMM) {

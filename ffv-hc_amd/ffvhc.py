@@ -321,6 +321,11 @@ class Context:
         it a launch of its own every iteration."""
         check(_L.ffvhc_ctx_set_option(self.h, 6, int(bool(on))), "ffvhc_ctx_set_option")
 
+    def set_resident(self, on):
+        """Run solves of at most 256 active blocks in one launch whose blocks stay on the chip (default), or
+        launch every stage of every iteration."""
+        check(_L.ffvhc_ctx_set_option(self.h, 7, int(bool(on))), "ffvhc_ctx_set_option")
+
     def set_classes(self, on):
         """Let the compact-record solve methods (11-28) read the bands of blocks that are uniform
         per stencil position class from 27 rows (default), or read every block per cell."""
