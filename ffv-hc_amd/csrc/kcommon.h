@@ -143,6 +143,14 @@ struct ColumnBands {
 __device__ inline double half_lo(uint32_t u) { return (double)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xffffu)); }
 __device__ inline double half_hi(uint32_t u) { return (double)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16)); }
 
+// The thread's index, opaque to the compiler: what a loop or stage derives from it (addresses, face
+// tests) is formed there and not carried in registers through the rest of the kernel.
+__device__ inline int thread_here() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // f(true_type) for a class-uniform block, f(false_type) else (uniform over the workgroup)
 template <class T, class F>
 __device__ inline void by_class(const ClassRows<T>& R, int slot, const F& f) {

@@ -25,6 +25,24 @@ enum FinalOp {
 void launch_finalize(hipStream_t sm, const int* caseact, int ncase, const DevCase* cs, SolveState* st,
                      const double* part, size_t nslots, int op, int arg, const SolveState* gate = nullptr);
 
+// ghost layers of n independent fields: values, ghosts, boundary condition group and updater of each
+template <class T>
+struct GhostFields {
+  static constexpr int MAX = 5;
+  int n = 0;
+  const T* x[MAX];
+  T* h[MAX];
+  int bcg[MAX], updater[MAX];
+  void add(const T* xf, T* hf, int group, int up) {
+    x[n] = xf;
+    h[n] = hf;
+    bcg[n] = group;
+    updater[n++] = up;
+  }
+};
+template <class T>
+void launch_ghost_pull(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
+                       const GhostFields<T>& fields, bool multilevel);
 template <class T>
 void launch_ghost_pull(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                        const T* x, T* h, int bcg, int updater, bool multilevel);

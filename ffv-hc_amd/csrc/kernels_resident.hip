@@ -56,14 +56,6 @@ struct PutDevice {
   }
 };
 
-// The thread's index, opaque to the compiler: what a stage derives from it (addresses, face tests) is
-// formed there and not carried in registers through the whole solve.
-__device__ inline int thread_here() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
-
 // a or b by value: the conditional operator on two array elements selects an address, which would put
 // the arrays in memory
 template <class T>

@@ -1826,10 +1826,14 @@ int ffvhc_step(ffvhc_ctx* c, ffvhc_step_fields* F, const ffvhc_step_params* P, f
   S.lapp = D(F->lapp);
   S.t = F->t < 0 ? nullptr : D(F->t);
   const size_t capnc = (size_t)c->cap * NC;
-  auto fill_u = [&]() {
-    for (int d = 0; d < 3; d++)
-      launch_ghost_pull<double>(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S.u[d], S.hu[d], BC_UX + d, 5,
-                                c->multilevel);
+  auto fill = [&](bool velocity, bool pressure) {  // the ghosts of u and of p and its Laplacian
+    GhostFields<double> G;
+    for (int d = 0; velocity && d < 3; d++) G.add(S.u[d], S.hu[d], BC_UX + d, 5);
+    if (pressure) {
+      G.add(S.p, S.hp, BC_P, 1);
+      G.add(S.lapp, H(F->lapp), BC_NULL, 1);
+    }
+    launch_ghost_pull<double>(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, G, c->multilevel);
   };
   hipEvent_t ev[4];
   for (auto& e : ev) HIPCHK(hipEventCreate(&e));
@@ -1846,18 +1850,17 @@ int ffvhc_step(ffvhc_ctx* c, ffvhc_step_fields* F, const ffvhc_step_params* P, f
       int stu = ffvhc_bicgstab(c, u[d], F->A, F->b, BC_UX + d, P->omega_u, 1, P->countMax_u, P->eps_u,
                                cntu.data() + d * nc, resu.data() + d * nc);
       if (stu < 0) return stu;
-      launch_ghost_pull<double>(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S.u[d], S.hu[d], BC_UX + d, 5,
-                                c->multilevel);
     }
+    fill(true, false);  // a component's matrix and RHS read no other component's ghosts
   } else {
     // UpdateUXe / UYe / UZe: the three components are independent (face velocities are fixed)
     launch_predict(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S, c->dcut, c->dflag, capnc);
-    fill_u();
+    fill(true, false);
   }
   HIPCHK(hipEventRecord(ev[1], c->sm));
   // UpdateP
   launch_p1(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S, c->dcut, c->dflag, capnc);
-  fill_u();
+  fill(true, false);
   launch_ab_p(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S, c->dcut, c->dflag, capnc);
   if (P->ref_active) {
     std::vector<int> cand;
@@ -1909,10 +1912,7 @@ int ffvhc_step(ffvhc_ctx* c, ffvhc_step_fields* F, const ffvhc_step_params* P, f
   HIPCHK(hipEventRecord(ev[2], c->sm));
   // UpdateU
   launch_corr(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S, c->dcut, c->dflag, capnc);
-  fill_u();
-  launch_ghost_pull<double>(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S.p, S.hp, BC_P, 1, c->multilevel);
-  launch_ghost_pull<double>(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, S.lapp, H(F->lapp), BC_NULL, 1,
-                            c->multilevel);
+  fill(true, true);
   HIPCHK(hipEventRecord(ev[3], c->sm));
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventSynchronize(ev[3]));

@@ -1,0 +1,47 @@
+"""The stage kernels' body for blocks without cut or solid cells, against the oracle, and the per-case
+extrema of more blocks than a workgroup has threads."""
+import numpy as np
+import pytest
+
+import ffvhc
+from helpers import G, N, OracleGrid, geometry
+from test_gpu_step import BC, ctx, run_case, trees  # noqa: F401 (ctx is a fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cut_blocks", [0, 1])
+@pytest.mark.parametrize("name", ["flat", "two_level"])
+@pytest.mark.parametrize("implicit", [None, (0.5, 1.0, 1e-30, 8)])
+def test_whole_blocks_match_oracle(ctx, name, cut_blocks, implicit):  # noqa: F811
+    """Bit for bit (explicit U; BiCGSTAB of the implicit one to rounding) with no cut block and with one
+    among whole ones."""
+    tree = trees()[name]
+    og = OracleGrid(tree)
+    geo = geometry(og, np.random.default_rng(11))
+    c, cid, pid = (x.copy() for x in geo)
+    for f in range(6):
+        c[f][cut_blocks:] = 1.0
+        cid[f][cut_blocks:] = 0
+    pid[cut_blocks:] = 1
+    run_case(ctx, name, solver=0, omega=1.2, count_max=20, eps=1e-30, tol=0.0 if implicit is None else 1e-9, nsteps=1,
+             implicit=implicit, tree=tree, geo=(c, cid, pid))
+
+
+@pytest.mark.parametrize("where", [0, 255, 256, -1])
+def test_stats_of_many_blocks(where):
+    """Extrema that lie in the first, the last of the first round, the next and the last block."""
+    tree = ffvhc.Tree(root=(8, 6, 6), root_length=1.0)
+    assert tree.nblk > 256
+    ctx = ffvhc.Context(max_blocks=tree.nblk)
+    try:
+        cid = ctx.add_case(tree, ffvhc.case_params(bc=BC))
+        f = ctx.field(8)
+        x = np.random.default_rng(3).uniform(0.5, 1.0, (tree.nblk, N, N, N))
+        x[where, 3, 5, 7], x[where, 15, 0, 15] = 2.0, -3.0
+        x[where, 0, 0, 0] = 1e-9
+        ctx.upload(f, cid, np.pad(x, ((0, 0),) + ((G, G),) * 3))
+        got = ctx.stats(f, ncases=1)[0]
+        assert list(got[1:]) == [2.0, -3.0, 3.0, 1e-9]
+    finally:
+        ctx.close()
