@@ -133,8 +133,8 @@ template <class T>
 void launch_bicgstab_restart(hipStream_t sm, const int* active, int nact, const DevBlock* blk, const SolveState* st,
                              BiVecs<T> V);
 // Resident solvers (kernels_resident.hip): one launch runs up to `turns` iterations of a solve whose
-// blocks (one workgroup each, at most RS_MAX) are on the chip together.
-constexpr int RS_MAX = 256;
+// blocks (one workgroup each) are on the chip together: at most RS_MAX, or RS_MAX2 two a compute unit.
+constexpr int RS_MAX = 256, RS_MAX2 = 512;
 constexpr int RS_COPIES = 8;                // copies of a block's words in a meeting
 constexpr int RS_WORDS = 9 * RS_COPIES + 1;  // 8-byte words per slot
 

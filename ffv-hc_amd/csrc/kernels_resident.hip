@@ -1,6 +1,8 @@
 // Solvers whose blocks stay on the chip: one launch runs a whole solve of up to one 16^3 block per
 // compute unit (BiCGSTAB: FFVILS.h:793-974, CG: 661-791, RBGS / Jacobi: 492-594), each workgroup
-// keeping its block's vectors in registers and LDS from the first iteration to the last.
+// keeping its block's vectors in registers and LDS from the first iteration to the last.  Jacobi
+// BiCGSTAB, CG, Jacobi and FP32 RBGS also run with two blocks per compute unit (PAIR), at half the
+// registers and LDS a block: vectors read once an iteration then stay in memory, which L2 serves.
 //
 // What bounds a small grid is not bytes but chains: with one launch per stage (kernels_bicg.hip,
 // kernels_cg.hip, kernels_core.hip) an iteration is five to seven launches of 7-15 us each at 16-128
@@ -29,6 +31,10 @@
 // blocks (of 32: two preconditioners 2 x 8, meetings 13), Jacobi BiCGSTAB 46 -> 21 us at 128 and 68 ->
 // 28 us at 256 blocks, PCG 26 -> 10 us at 60, RBGS 14 -> 8.6 us and Jacobi 13.4 -> 7.9 us at 128.  A
 // meeting of everyone takes 2.4 us with 16 workgroups and 3.4-4 with 128, one of neighbours 1.4-2.
+// PAIR, a solve: Jacobi BiCGSTAB 48.5 -> 25.7 ms at 288 and 59.7 -> 32.7 ms at 512 blocks, PCG 35.4 -> 20.9
+// and 53.2 -> 28.1 ms, 100 Jacobi sweeps 1.81 -> 1.43 and 2.16 -> 1.83 ms.  With x, r0 and the diagonal in
+// registers as in the other form the compiler spilled 56-193 of 128 registers (CG 1.1x); what every lane
+// has in scalar registers (scalar()) took 26-46 spills out of each kernel.
 #include "kcommon.h"
 #include "kernels.h"
 
@@ -36,10 +42,12 @@ namespace ffvhc {
 
 constexpr int RS_NT = 512;                // two threads per (i, j) column, 8 cells each
 constexpr int RS_NK = NB * NF / RS_NT;    // cells per thread
-constexpr int RS_EN = RS_MAX / 64;        // words of one kind a lane reads in a meeting
 constexpr unsigned long long kUnset = 0x7FF0DEADBEEF0001ull;
 constexpr unsigned long long kWaitTicks = 400000000ull;  // 4 s of the 100 MHz clock
 static_assert(RS_NK == 8 && RS_MAX % 256 == 0, "layout of the reductions below");
+// words of one kind a lane reads in a meeting, with one or two workgroups a compute unit (PAIR)
+template <bool PAIR>
+constexpr int kWords = (PAIR ? RS_MAX2 : RS_MAX) / 64;
 
 template <class T>
 __device__ inline T load_device(const T* p) {
@@ -61,6 +69,18 @@ struct PutDevice {
 template <class T>
 __device__ inline T pick(bool c, T a, T b) {
   return c ? a : b;
+}
+
+// a value that every lane has, in scalar registers (a struct of 8-byte and 4-byte members too)
+template <class V>
+__device__ inline V scalar(V v) {
+  static_assert(sizeof(V) % 4 == 0);
+  uint32_t w[sizeof(V) / 4];
+  __builtin_memcpy(w, &v, sizeof(V));
+#pragma unroll
+  for (size_t q = 0; q < sizeof(V) / 4; q++) w[q] = __builtin_amdgcn_readfirstlane(w[q]);
+  __builtin_memcpy(&v, w, sizeof(V));
+  return v;
 }
 
 // Scratch of the meetings in LDS: partial sums by wavefront, results, the mark of a wait that ended
@@ -85,7 +105,7 @@ struct Meeting {
   // blocks lane + 64 m (0 past n).  Each workgroup writes its words RS_COPIES times and reads one copy,
   // so that few poll the same cache line (128 workgroups, one copy: 4.2 us a meeting).  False: a wait
   // ended without everyone (uniform over the workgroup).
-  template <int NP, int NW = 4, int NW2 = NW, class Use>
+  template <int NP, int EN, int NW = 4, int NW2 = NW, class Use>
   __device__ bool all(MeetLds& M, const Use& use) {
     const int t = thread_here(), lane = t & 63;
     // this wavefront's stores have arrived: ghosts, and the words it unset in the last meeting
@@ -100,25 +120,25 @@ struct Meeting {
     const int k = t >> 6;
     if (k < NP) {
       const unsigned long long* const w = word(epoch, k, blockIdx.x % RS_COPIES) + begin;
-      unsigned long long b[RS_EN];
+      unsigned long long b[EN];
 #pragma unroll
-      for (int m = 0; m < RS_EN; m++) b[m] = lane + 64 * m < n ? kUnset : 0ull;
+      for (int m = 0; m < EN; m++) b[m] = lane + 64 * m < n ? kUnset : 0ull;
       const unsigned long long t0 = wall_clock64();
       bool there = false;
       while (!there) {
         bool here = true;
 #pragma unroll
-        for (int m = 0; m < RS_EN; m++)
+        for (int m = 0; m < EN; m++)
           if (b[m] == kUnset) b[m] = load_device(w + lane + 64 * m);
 #pragma unroll
-        for (int m = 0; m < RS_EN; m++) here = here && b[m] != kUnset;
+        for (int m = 0; m < EN; m++) here = here && b[m] != kUnset;
         there = __all(here);
         if (!there && wall_clock64() - t0 > kWaitTicks) break;
       }
       if (there) {
-        double e[RS_EN];
+        double e[EN];
 #pragma unroll
-        for (int m = 0; m < RS_EN; m++) e[m] = __longlong_as_double((long long)b[m]);
+        for (int m = 0; m < EN; m++) e[m] = __longlong_as_double((long long)b[m]);
         use(k, e);
         if (t < 3 * RS_COPIES && epoch > 0)
           store_device(word(epoch - 1, t / RS_COPIES, t % RS_COPIES) + slot, kUnset);
@@ -157,23 +177,25 @@ struct Meeting {
 };
 
 // the sum over the case in the order of the per-case finalisation (case_sum)
-__device__ inline double case_order(const double* e) {
+template <int EN>
+__device__ inline double case_order(const double (&e)[EN]) {
   double s = 0.0;
 #pragma unroll
   for (int w = 0; w < 4; w++) {
     double v = 0.0;
 #pragma unroll
-    for (int m = w; m < RS_EN; m += 4) v += e[m];
+    for (int m = w; m < EN; m += 4) v += e[m];
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     s += v;
   }
   return s;
 }
 // ... and in that of the coarse application's alpha (one wavefront, lane-strided)
-__device__ inline double lane_order(const double* e) {
+template <int EN>
+__device__ inline double lane_order(const double (&e)[EN]) {
   double v = 0.0;
 #pragma unroll
-  for (int m = 0; m < RS_EN; m++) v += e[m];
+  for (int m = 0; m < EN; m++) v += e[m];
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
@@ -389,12 +411,20 @@ __device__ inline void push_faces(const FaceLds& F, int slot, const Acc& L, cons
 // meetings carry along.
 //   per iteration: P meet Q meet S meet T meet XR meet
 // ------------------------------------------------------------------------------------------
-template <bool TWO>
-__global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a) {
+// PAIR (two workgroups a compute unit, Jacobi): 128 registers a thread and 80 KB of LDS.  x and r0 stay
+// in memory (32 KB a block, from L2), q_ goes to LDS, p_ is formed again where it is added to x, and the
+// columns' partial sums take the place of the ghosts that the matvec has read.
+template <bool TWO, bool PAIR>
+__global__ __launch_bounds__(RS_NT, PAIR ? 4 : 2) void resident_bicg_kernel(ResidentBicg a) {
+  static_assert(!(TWO && PAIR));
   using TM = std::conditional_t<TWO, float, double>;
+  constexpr int EN = kWords<PAIR>;
   __shared__ Operand<double> Z;
-  __shared__ double xs[NC], r0s[NC];  // x and r0: read once or twice an iteration, so LDS holds them
-  __shared__ double chain[3][NF];
+  // x and r0: read once or twice an iteration, so LDS holds them
+  __shared__ double xs[PAIR ? 1 : NC], r0s[PAIR ? 1 : NC], qs[PAIR ? NC : 1];
+  __shared__ double chains[PAIR ? 1 : 3][NF];
+  double(*const chain)[NF] = PAIR ? reinterpret_cast<double(*)[NF]>(Z.side) : chains;
+  static_assert(4 * NF >= 3 * NF);
   __shared__ MeetLds L;
   // TWO: block sums of r, q_, p over the case, the coarse right-hand side, and the corrections of
   // this block (0) and of the blocks its ghosts come from (near.at[4 face + quarter])
@@ -405,7 +435,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
   const int slot = a.active[blockIdx.x];
   const DevBlock& B = a.blk[slot];
   const int c = B.case_id;
-  SolveState S = a.st[c];
+  SolveState S = scalar(a.st[c]);
   if (S.done) return;
   const DevCase& C = a.cs[c];
   const int t = threadIdx.x, tx = t & 15, ty = (t >> 4) & 15, kb = (t >> 8) * RS_NK, lane = t & 63;
@@ -455,10 +485,14 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
 #pragma unroll
   for (int k = 0; k < RS_NK; k++) {
     r[k] = a.V.r[g0 + NF * k];
-    r0s[l0 - NF + NF * k] = a.V.r0[g0 + NF * k];
-    xs[l0 - NF + NF * k] = a.x[g0 + NF * k];
     p[k] = S.iter ? a.V.p[g0 + NF * k] : 0.0;
     q[k] = S.iter ? a.V.q[g0 + NF * k] : 0.0;
+    if constexpr (PAIR) {
+      qs[l0 - NF + NF * k] = q[k];
+    } else {
+      r0s[l0 - NF + NF * k] = a.V.r0[g0 + NF * k];
+      xs[l0 - NF + NF * k] = a.x[g0 + NF * k];
+    }
   }
   __syncthreads();
 
@@ -475,7 +509,8 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
       for (int i = 0; i < CR; i++) {
         const int e = (u >> 6) + i * (RS_NT / 64);
         if (e < near.n && 4 * (u & 63) < np)
-          crow[i] = reinterpret_cast<const float4*>(a.cinv + a.coff[c] + (size_t)(near.slot[e] - C.slot_begin) * np)[u & 63];
+          crow[i] = reinterpret_cast<const float4*>(a.cinv + a.coff[c] +
+                                                    (size_t)(near.slot[e] - C.slot_begin) * np)[u & 63];
       }
     }
   };
@@ -507,6 +542,19 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
     }
   };
 
+  // !TWO: to(k, omega v / Ap) for the thread's cells
+  auto jacobi = [&](const double (&v)[RS_NK], const auto& to) __attribute__((always_inline)) {
+    const int t = thread_here(), tx = t & 15, ty = (t >> 4) & 15, kb = (t >> 8) * RS_NK;
+    const bool lower = kb == 0;
+    const TM* tr = class_column(R.tab, slot, tx, ty);
+    const double din = R.uni ? (double)tr[9 * 8] : 0.0, dend = R.uni ? (double)tr[lower ? 0 : 18 * 8] : 0.0;
+#pragma unroll
+    for (int k = 0; k < RS_NK; k++) {
+      double d = k == 0 ? (lower ? dend : din) : k == RS_NK - 1 ? (lower ? din : dend) : din;
+      if ((ex >> k) & 1u) d = A.p[0][(size_t)slot * NC + tx + NB * ty + NF * (kb + k)];
+      to(k, omega * (v[k] / d));
+    }
+  };
   // z = M v into Z.zpad (bi_precond_kernel / bi_precond_gsk_kernel), its ghosts pushed to h
   auto precond = [&](const double (&v)[RS_NK], double* h) __attribute__((always_inline)) {
     const int t = thread_here(), tx = t & 15, ty = (t >> 4) & 15, kb = (t >> 8) * RS_NK;
@@ -515,14 +563,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
     const int l0 = tx + NB * ty + NF * (kb + 1);
     double* const z = Z.zpad + NF;
     if constexpr (!TWO) {
-      const double* tr = class_column(R.tab, slot, tx, ty);
-      const double din = R.uni ? tr[9 * 8] : 0.0, dend = R.uni ? tr[lower ? 0 : 18 * 8] : 0.0;
-#pragma unroll
-      for (int k = 0; k < RS_NK; k++) {
-        double d = k == 0 ? (lower ? dend : din) : k == RS_NK - 1 ? (lower ? din : dend) : din;
-        if ((ex >> k) & 1u) d = A.p[0][g0 + NF * k];
-        Z.zpad[l0 + NF * k] = omega * (v[k] / d);
-      }
+      jacobi(v, [&](int k, double z) { Z.zpad[l0 + NF * k] = z; });
     } else {
       const double eo = ev[0], ex_ = ev[ix], ey = ev[iy], ez = ev[iz];
       const int par = (tx + ty) & 1;
@@ -634,14 +675,18 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
     half_matvec<double, TM>(Z, W, A, ex, (size_t)slot * NC + ux + NB * uy + NF * uk, ux, uy, uk, y);
   };
   auto keep = [&](double* to) {  // a word of every block into LDS
-    return [=](const double* e) {
+    return [=](const double (&e)[EN]) {
       const int lane = thread_here() & 63;
 #pragma unroll
-      for (int m = 0; m < RS_EN; m++)
+      for (int m = 0; m < EN; m++)
         if (lane + 64 * m < nn) to[lane + 64 * m] = e[m];
     };
   };
 
+  auto shadow = [&]() -> const double* {
+    if constexpr (PAIR) return a.V.r0 + (size_t)slot * NC;
+    return r0s;
+  };
   FinXr f = {};
   double alpha = S.alpha, beta = S.beta, gamma = S.gamma, rho = S.rr1, rho_n = rho;
   int n = S.iter;
@@ -658,12 +703,14 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
     double vs = 0.0;
 #pragma unroll
     for (int k = 0; k < RS_NK; k++) {
-      p[k] = first ? r[k] : r[k] + beta * (p[k] + ng * q[k]);
+      const double qk = PAIR ? qs[l0 - NF + NF * k] : q[k];
+      p[k] = first ? r[k] : r[k] + beta * (p[k] + ng * qk);
       vs += p[k];
     }
     precond(p, a.V.hpp);
+    if constexpr (!PAIR)
 #pragma unroll
-    for (int k = 0; k < RS_NK; k++) pp[k] = Z.zpad[l0 + NF * k];
+      for (int k = 0; k < RS_NK; k++) pp[k] = Z.zpad[l0 + NF * k];
     if constexpr (TWO) {
       for (int o = 32; o > 0; o >>= 1) vs += __shfl_xor(vs, o, 64);
       if ((thread_here() & 63) == 0) L.red[2][thread_here() >> 6] = vs;  // goes out with q_'s sums
@@ -672,17 +719,21 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
     if (!ok) break;
     // Q
     matvec(a.V.hpp, q);
+    if constexpr (PAIR) __syncthreads();  // the ghosts have been read
     column_sums<2>(chain, L, [&](double* v) {
       const int u = thread_here();  // the thread's cells are u + 256 k in xs and r0s, from the half's base on
-      const double* const r0 = r0s + (u & (NF - 1)) + (u >> 8) * RS_NK * NF;
+      const double* const r0 = shadow() + (u & (NF - 1)) + (u >> 8) * RS_NK * NF;
 #pragma unroll
       for (int k = 0; k < RS_NK; k++) {
         v[0] += q[k] * r0[NF * k];
         v[1] += q[k];
       }
     });
+    if constexpr (PAIR)
+#pragma unroll
+      for (int k = 0; k < RS_NK; k++) qs[l0 - NF + NF * k] = q[k];
     coarse_load();
-    ok = meet.template all<TWO ? 3 : 1, 4, RS_NT / 64>(L, [&](int k, const double* e) {
+    ok = meet.template all<TWO ? 3 : 1, EN, 4, RS_NT / 64>(L, [&](int k, const double (&e)[EN]) {
       if (k == 1)
         keep(bq)(e);
       else if (k == 2)
@@ -693,18 +744,19 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
       }
     });
     if (!ok) break;
-    alpha = rho / L.sum[0];
+    alpha = scalar(rho / L.sum[0]);
     const double na = -alpha;
     // S (r becomes s)
     coarse_rhs([&](int b) { return na * bq[b] + br[b]; });
     coarse();
 #pragma unroll
-    for (int k = 0; k < RS_NK; k++) r[k] = na * q[k] + r[k];
+    for (int k = 0; k < RS_NK; k++) r[k] = na * (PAIR ? qs[l0 - NF + NF * k] : q[k]) + r[k];
     precond(r, a.V.hss);
     ok = meet.neighbours(L, near.slot, near.n);
     if (!ok) break;
     // T
     matvec(a.V.hss, tt);
+    if constexpr (PAIR) __syncthreads();
     column_sums<2>(chain, L, [&](double* v) {
 #pragma unroll
       for (int k = 0; k < RS_NK; k++) {
@@ -712,26 +764,32 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
         v[1] += tt[k] * tt[k];
       }
     });
-    ok = meet.template all<2>(L, [&](int k, const double* e) {
+    ok = meet.template all<2, EN>(L, [&](int k, const double (&e)[EN]) {
       const double s = case_order(e);
       if (lane == 0) L.sum[k] = s;
     });
     if (!ok) break;
-    gamma = L.sum[0] / L.sum[1];
+    gamma = scalar(L.sum[0] / L.sum[1]);
     const double mg = -gamma;
     // XR
     {
       const int u = thread_here(), own = (u & (NF - 1)) + (u >> 8) * RS_NK * NF;
+      double* const xb = PAIR ? a.x + (size_t)slot * NC : xs;
+      auto add = [&](int k, double pk) {
+        double& x = xb[own + NF * k];
+        x = alpha * pk + gamma * Z.zpad[NF + own + NF * k] + x;  // s_ is still there
+      };
+      if constexpr (PAIR)
+        jacobi(p, add);
+      else
 #pragma unroll
-      for (int k = 0; k < RS_NK; k++) {
-        double& x = xs[own + NF * k];
-        x = alpha * pp[k] + gamma * Z.zpad[NF + own + NF * k] + x;  // s_ is still there
-        r[k] = mg * tt[k] + r[k];
-      }
+        for (int k = 0; k < RS_NK; k++) add(k, pp[k]);
+#pragma unroll
+      for (int k = 0; k < RS_NK; k++) r[k] = mg * tt[k] + r[k];
     }
     column_sums<3>(chain, L, [&](double* v) {
       const int u = thread_here();
-      const double* const r0 = r0s + (u & (NF - 1)) + (u >> 8) * RS_NK * NF;
+      const double* const r0 = shadow() + (u & (NF - 1)) + (u >> 8) * RS_NK * NF;
 #pragma unroll
       for (int k = 0; k < RS_NK; k++) {
         v[2] += r[k];
@@ -740,7 +798,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
       }
     });
     coarse_load();
-    ok = meet.template all<TWO ? 3 : 2>(L, [&](int k, const double* e) {
+    ok = meet.template all<TWO ? 3 : 2, EN>(L, [&](int k, const double (&e)[EN]) {
       if (k == 2)
         keep(br)(e);
       else {
@@ -752,7 +810,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
     S.alpha = alpha;
     S.gamma = gamma;
     rho_n = rho;
-    f = fin_bi_xr_eval(S, L.sum[0], L.sum[1], n, rho_n);
+    f = scalar(fin_bi_xr_eval(S, L.sum[0], L.sum[1], n, rho_n));
     rho = f.rr1;
     beta = f.beta;
     if (f.done || n >= stop) break;
@@ -763,11 +821,11 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
   }
 #pragma unroll
   for (int k = 0; k < RS_NK; k++) {
-    a.x[g0 + NF * k] = xs[l0 - NF + NF * k];
+    if constexpr (!PAIR) a.x[g0 + NF * k] = xs[l0 - NF + NF * k];
     if (!f.done) {  // to be continued by the next launch
       a.V.r[g0 + NF * k] = r[k];
       a.V.p[g0 + NF * k] = p[k];
-      a.V.q[g0 + NF * k] = q[k];
+      a.V.q[g0 + NF * k] = PAIR ? qs[l0 - NF + NF * k] : q[k];
     }
   }
   if (TWO && t == 0 && !f.done) {
@@ -786,8 +844,10 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_bicg_kernel(ResidentBicg a)
 // ------------------------------------------------------------------------------------------
 // Jacobi-PCG after its initialisation (r, b.b and r.z are there): P neighbours Q meet XR meet
 // ------------------------------------------------------------------------------------------
-template <class T>
-__global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) {
+// PAIR: x stays in memory, z and Ap are formed where they are used.
+template <class T, bool PAIR>
+__global__ __launch_bounds__(RS_NT, PAIR ? 4 : 2) void resident_cg_kernel(ResidentCg<T> a) {
+  constexpr int EN = kWords<PAIR>;
   __shared__ Operand<T> Z;
   __shared__ double chain[2][NF];
   __shared__ MeetLds L;
@@ -796,7 +856,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) 
   const int slot = a.active[blockIdx.x];
   const DevBlock& B = a.blk[slot];
   const int c = B.case_id;
-  SolveState S = a.st[c];
+  SolveState S = scalar(a.st[c]);
   if (S.done) return;
   const DevCase& C = a.cs[c];
   const int t = threadIdx.x, tx = t & 15, ty = (t >> 4) & 15, kb = (t >> 8) * RS_NK, lane = t & 63;
@@ -811,19 +871,30 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) 
   const T omega = (T)S.omega;
   const unsigned ex = a.R.uni ? a.R.ex[(size_t)slot * 512 + t] : 0xffu;
   T x[RS_NK], r[RS_NK], p[RS_NK], z[RS_NK], d[RS_NK];  // d: Ap
-  {
+  // to(k, Ap) for the thread's cells
+  auto diagonal = [&](const auto& to) __attribute__((always_inline)) {
+    const int t = thread_here(), tx = t & 15, ty = (t >> 4) & 15, kb = (t >> 8) * RS_NK;
+    const bool lower = kb == 0;
     const T* tr = class_column(a.R.tab, slot, tx, ty);
     const T din = a.R.uni ? tr[9 * 8] : (T)0, dend = a.R.uni ? tr[lower ? 0 : 18 * 8] : (T)0;
 #pragma unroll
     for (int k = 0; k < RS_NK; k++) {
-      x[k] = a.x[g0 + NF * k];
-      r[k] = a.r[g0 + NF * k];
-      p[k] = S.iter ? a.p[g0 + NF * k] : (T)0;
-      d[k] = k == 0 ? pick(lower, dend, din) : k == RS_NK - 1 ? pick(lower, din, dend) : din;
-      if ((ex >> k) & 1u) d[k] = a.A.p[0][g0 + NF * k];
-      z[k] = omega * (r[k] / d[k]);
+      T v = k == 0 ? pick(lower, dend, din) : k == RS_NK - 1 ? pick(lower, din, dend) : din;
+      if ((ex >> k) & 1u) v = a.A.p[0][(size_t)slot * NC + tx + NB * ty + NF * (kb + k)];
+      to(k, v);
     }
+  };
+#pragma unroll
+  for (int k = 0; k < RS_NK; k++) {
+    if constexpr (!PAIR) x[k] = a.x[g0 + NF * k];
+    r[k] = a.r[g0 + NF * k];
+    p[k] = S.iter ? a.p[g0 + NF * k] : (T)0;
   }
+  if constexpr (!PAIR)
+    diagonal([&](int k, T v) {
+      d[k] = v;
+      z[k] = omega * (r[k] / v);
+    });
   __syncthreads();
   const int stop = S.iter + a.turns;
   bool ok = true;
@@ -832,11 +903,15 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) 
     const T beta = (T)S.beta;
     {
       const int u = thread_here(), own = (u & (NF - 1)) + NF * ((u >> 8) * RS_NK + 1);
-#pragma unroll
-      for (int k = 0; k < RS_NK; k++) {
-        p[k] = n == 1 ? z[k] : z[k] + beta * p[k];
+      auto step = [&](int k, T zk) {
+        p[k] = n == 1 ? zk : zk + beta * p[k];
         Z.zpad[own + NF * k] = p[k];
-      }
+      };
+      if constexpr (PAIR)
+        diagonal([&](int k, T v) { step(k, omega * (r[k] / v)); });
+      else
+#pragma unroll
+        for (int k = 0; k < RS_NK; k++) step(k, z[k]);
     }
     __syncthreads();
     push_faces<T>(faces, slot, [&](int i, int j, int k) { return Z.zpad[NF + i + NB * (j + NB * k)]; }, a.hp, a.hp);
@@ -856,19 +931,26 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) 
 #pragma unroll
       for (int k = 0; k < RS_NK; k++) v[0] += (double)q[k] * (double)p[k];
     });
-    ok = meet.template all<1>(L, [&](int, const double* e) {
+    ok = meet.template all<1, EN>(L, [&](int, const double (&e)[EN]) {
       const double s = case_order(e);
       if (lane == 0) L.sum[0] = s;
     });
     if (!ok) break;
-    S.alpha = S.rr1 / L.sum[0];
+    S.alpha = scalar(S.rr1 / L.sum[0]);
     const T alpha = (T)S.alpha, nalpha = -alpha;
     // XR
 #pragma unroll
     for (int k = 0; k < RS_NK; k++) {
-      x[k] = x[k] + alpha * p[k];
+      if constexpr (!PAIR) x[k] = x[k] + alpha * p[k];
       r[k] = r[k] + nalpha * q[k];
-      z[k] = omega * (r[k] / d[k]);
+      if constexpr (!PAIR) z[k] = omega * (r[k] / d[k]);
+    }
+    if constexpr (PAIR) {
+      const int u = thread_here();
+      T* const xb = a.x + (size_t)slot * NC + (u & (NF - 1)) + (u >> 8) * RS_NK * NF;
+#pragma unroll
+      for (int k = 0; k < RS_NK; k++) xb[NF * k] = xb[NF * k] + alpha * p[k];
+      diagonal([&](int k, T v) { z[k] = omega * (r[k] / v); });
     }
     column_sums<2>(chain, L, [&](double* v) {
 #pragma unroll
@@ -877,13 +959,14 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) 
         v[1] += (double)r[k] * (double)z[k];
       }
     });
-    ok = meet.template all<2>(L, [&](int k, const double* e) {
+    ok = meet.template all<2, EN>(L, [&](int k, const double (&e)[EN]) {
       const double s = case_order(e);
       if (lane == 0) L.sum[k] = s;
     });
     if (!ok) break;
     S.iter = n;
     cg_end(S, L.sum[0], L.sum[1], n);
+    S = scalar(S);
     if (S.done || n >= stop) break;
   }
   if (!ok) {
@@ -892,7 +975,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) 
   }
 #pragma unroll
   for (int k = 0; k < RS_NK; k++) {
-    a.x[g0 + NF * k] = x[k];
+    if constexpr (!PAIR) a.x[g0 + NF * k] = x[k];
     if (!S.done) {  // to be continued by the next launch
       a.r[g0 + NF * k] = r[k];
       a.p[g0 + NF * k] = p[k];
@@ -904,10 +987,11 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_cg_kernel(ResidentCg<T> a) 
 // ------------------------------------------------------------------------------------------
 // RBGS (MODE 0) and Jacobi (MODE 1): iteration n sweeps x^{n-1} to x^n, pushes its ghosts into the
 // other halo buffer and meets over the residual of x^{n-1} (rbgs_iter_kernel).  The result, x and
-// its ghosts, goes to buffer 0.
+// its ghosts, goes to buffer 0.  PAIR: b stays in memory and the bands are read again each iteration.
 // ------------------------------------------------------------------------------------------
-template <class T, int MODE>
-__global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<T> a) {
+template <class T, int MODE, bool PAIR>
+__global__ __launch_bounds__(RS_NT, PAIR ? 4 : 2) void resident_relax_kernel(ResidentRelax<T> a) {
+  constexpr int EN = kWords<PAIR>;
   __shared__ Operand<T> Z;
   __shared__ MeetLds L;
   __shared__ FaceLds faces;
@@ -915,7 +999,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
   const int slot = a.active[blockIdx.x];
   const DevBlock& B = a.blk[slot];
   const int c = B.case_id;
-  SolveState S = a.st[c];
+  SolveState S = scalar(a.st[c]);
   if (S.done) return;
   const DevCase& C = a.cs[c];
   const int t = threadIdx.x, tx = t & 15, ty = (t >> 4) & 15, kb = (t >> 8) * RS_NK, lane = t & 63;
@@ -929,15 +1013,17 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
   faces.load(B, C, a.bcg);
   const T omega = (T)S.omega;
   const unsigned ex = a.R.uni ? a.R.ex[(size_t)slot * 512 + t] : 0xffu;
-  T x[RS_NK], b[RS_NK], d[RS_NK];  // d: Ap
+  T x[RS_NK], bv[RS_NK], dv[RS_NK];
   HalfRows<T> W;
-  W.load(a.R, slot, tx, ty, lower);
+  if constexpr (!PAIR) W.load(a.R, slot, tx, ty, lower);
 #pragma unroll
   for (int k = 0; k < RS_NK; k++) {
     x[k] = a.x[g0 + NF * k];
-    b[k] = a.b[g0 + NF * k];
-    d[k] = k == 0 ? pick(lower, W.end[0], W.in[0]) : k == RS_NK - 1 ? pick(lower, W.in[0], W.end[0]) : W.in[0];
-    if ((ex >> k) & 1u) d[k] = a.A.p[0][g0 + NF * k];
+    if constexpr (!PAIR) {
+      bv[k] = a.b[g0 + NF * k];
+      dv[k] = k == 0 ? pick(lower, W.end[0], W.in[0]) : k == RS_NK - 1 ? pick(lower, W.in[0], W.end[0]) : W.in[0];
+      if ((ex >> k) & 1u) dv[k] = a.A.p[0][g0 + NF * k];
+    }
     Z.zpad[tx + NB * ty + NF * (kb + k + 1)] = x[k];
   }
   __syncthreads();
@@ -948,6 +1034,18 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
   for (int n = S.iter + 1;; n++) {
     const int u = thread_here(), ux = u & 15, uy = (u >> 4) & 15, uk = (u >> 8) * RS_NK;
     const size_t g = (size_t)slot * NC + ux + NB * uy + NF * uk;
+    if constexpr (PAIR) W.load(a.R, slot, ux, uy, uk == 0);
+    auto b = [&](int kk) -> T {
+      if constexpr (PAIR) return a.b[g + NF * kk];
+      return bv[kk];
+    };
+    auto d = [&](int kk) -> T {  // Ap
+      if constexpr (!PAIR) return dv[kk];
+      const T v = kk == 0 ? pick(uk != 0, W.in[0], W.end[0])
+                          : kk == RS_NK - 1 ? pick(uk != 0, W.end[0], W.in[0]) : W.in[0];
+      if ((ex >> kk) & 1u) return a.A.p[0][g + NF * kk];
+      return v;
+    };
     // b less the six neighbour products of cell kk with the bands w
     auto off_sum = [&](T bk, const T* w, int kk) -> T {
       const auto v = Z.around(ux, uy, uk + kk, ux + NB * uy + NF * (uk + kk + 1));
@@ -965,17 +1063,17 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
       T w[7];
 #pragma unroll
       for (int q = 1; q < 7; q++)
-        w[q] = kk == 0 ? pick(uk != 0, W.in[q], W.end[q]) : kk == RS_NK - 1 ? pick(uk != 0, W.end[q], W.in[q]) : W.in[q];
-      rs[kk] = off_sum(b[kk], w, kk);
+        w[q] = kk == 0 ? pick(uk != 0, W.in[q], W.end[q])
+                       : kk == RS_NK - 1 ? pick(uk != 0, W.end[q], W.in[q]) : W.in[q];
+      rs[kk] = off_sum(b(kk), w, kk);
       if (kk & 1) __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll 1
     for (unsigned m = ex; m; m &= m - 1) {
       const int kk = __builtin_ctz(m);
-      T w[7], bk = b[0];
+      T w[7];
       own_bands(w, kk);
-#pragma unroll
-      for (int k = 1; k < RS_NK; k++) bk = k == kk ? b[k] : bk;
+      const T bk = a.b[g + NF * kk];
       const T v = off_sum(bk, w, kk);
 #pragma unroll
       for (int k = 0; k < RS_NK; k++) rs[k] = k == kk ? v : rs[k];
@@ -983,16 +1081,16 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
     double sums[2] = {0.0, 0.0};
 #pragma unroll
     for (int kk = 0; kk < RS_NK; kk++) {
-      const T r = rs[kk] - d[kk] * x[kk];
+      const T r = rs[kk] - d(kk) * x[kk];
       sums[0] += (double)r * (double)r;
-      if (n == 1) sums[1] += (double)b[kk] * (double)b[kk];
+      if (n == 1) sums[1] += (double)b(kk) * (double)b(kk);
     }
     wave_sums<2>(sums, L, u >> 6);
     if (n <= S.countMax) {
       const int own = (u & (NF - 1)) + NF * (uk + 1);
       if constexpr (MODE == 1) {
 #pragma unroll
-        for (int kk = 0; kk < RS_NK; kk++) xn[kk] = x[kk] - omega * (x[kk] - rs[kk] / d[kk]);
+        for (int kk = 0; kk < RS_NK; kk++) xn[kk] = x[kk] - omega * (x[kk] - rs[kk] / d(kk));
         __syncthreads();
 #pragma unroll
         for (int kk = 0; kk < RS_NK; kk++) Z.zpad[own + NF * kk] = xn[kk];
@@ -1003,7 +1101,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
 #pragma unroll
         for (int m = 0; m < RS_NK / 2; m++) {
           const T xp = pick(par != 0, x[2 * m + 1], x[2 * m]);
-          xr[m] = xp - omega * (xp - pick(par != 0, rs[2 * m + 1], rs[2 * m]) / pick(par != 0, d[2 * m + 1], d[2 * m]));
+          xr[m] = xp - omega * (xp - pick(par != 0, rs[2 * m + 1], rs[2 * m]) / pick(par != 0, d(2 * m + 1), d(2 * m)));
         }
         __syncthreads();
 #pragma unroll
@@ -1016,15 +1114,14 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
           T w[7];
 #pragma unroll
           for (int q = 1; q < 7; q++) w[q] = pick(e, W.end[q], W.in[q]);
-          sb[m] = off_sum(pick(par != 0, b[2 * m], b[2 * m + 1]), w, 2 * m + 1 - par);
+          sb[m] = off_sum(pick(par != 0, b(2 * m), b(2 * m + 1)), w, 2 * m + 1 - par);
         }
 #pragma unroll 1
         for (unsigned mm = ex & (par ? 0x55u : 0xaau); mm; mm &= mm - 1) {
           const int kk = __builtin_ctz(mm);
-          T w[7], bk = b[0];
+          T w[7];
           own_bands(w, kk);
-#pragma unroll
-          for (int k = 1; k < RS_NK; k++) bk = k == kk ? b[k] : bk;
+          const T bk = a.b[g + NF * kk];
           const T v = off_sum(bk, w, kk);
 #pragma unroll
           for (int m = 0; m < RS_NK / 2; m++) sb[m] = m == kk >> 1 ? v : sb[m];
@@ -1032,7 +1129,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
 #pragma unroll
         for (int m = 0; m < RS_NK / 2; m++) {
           const T xb = pick(par != 0, x[2 * m], x[2 * m + 1]);
-          const T v = xb - omega * (xb - sb[m] / pick(par != 0, d[2 * m], d[2 * m + 1]));
+          const T v = xb - omega * (xb - sb[m] / pick(par != 0, d(2 * m), d(2 * m + 1)));
           xn[2 * m] = pick(par != 0, v, xr[m]);
           xn[2 * m + 1] = pick(par != 0, xr[m], v);
           Z.zpad[own + NF * (2 * m + 1 - par)] = v;
@@ -1042,7 +1139,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
       push_faces<T>(faces, slot, [&](int i, int j, int k) { return Z.zpad[NF + i + NB * (j + NB * k)]; }, a.h[cur],
                     a.h[cur ^ 1]);
     }
-    ok = meet.template all<2, RS_NT / 64>(L, [&](int k, const double* e) {
+    ok = meet.template all<2, EN, RS_NT / 64>(L, [&](int k, const double (&e)[EN]) {
       const double s = case_order(e);
       if (lane == 0) L.sum[k] = s;
     });
@@ -1055,6 +1152,7 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
     } else {
       converged(S, L.sum[0], n - 1);
     }
+    S = scalar(S);
     if (S.done) break;  // x^{n-1} and the ghosts it was read with are the result
 #pragma unroll
     for (int k = 0; k < RS_NK; k++) x[k] = xn[k];
@@ -1079,11 +1177,17 @@ __global__ __launch_bounds__(RS_NT, 2) void resident_relax_kernel(ResidentRelax<
   if (t == 0 && slot == C.slot_begin) a.st[c] = S;
 }
 
-// One workgroup per block of the active cases, at most RS_MAX; false: they do not fit on the device
-// together (or the launch is refused), nothing was launched.
+// One workgroup per block of the active cases; kernels[0] with one workgroup a compute unit, for up to
+// RS_MAX blocks, kernels[1] with two, for up to RS_MAX2 (limit[0], limit[1]: how many the device holds, -1
+// not asked yet).  False: they do not fit on the device together, there is no such kernel, or the launch is
+// refused; nothing was launched.
 template <class Args>
-bool launch_resident(const void* kernel, hipStream_t sm, int nact, int* limit, Args& args) {
-  if (nact < 1 || nact > RS_MAX) return false;
+bool launch_resident(const void* const (&kernels)[2], hipStream_t sm, int nact, int* limits, Args& args) {
+  if (nact < 1 || nact > RS_MAX2) return false;
+  const int pair = nact > RS_MAX;
+  const void* const kernel = kernels[pair];
+  if (!kernel) return false;
+  int* const limit = limits + pair;
   if (*limit < 0) {
     int per = 0, dev = 0, cus = 0, coop = 0;
     *limit = 0;
@@ -1105,19 +1209,29 @@ bool launch_resident(const void* kernel, hipStream_t sm, int nact, int* limit, A
   return true;
 }
 
-bool launch_resident_bicg(hipStream_t sm, int nact, bool two, int* limit, ResidentBicg& args) {
-  const void* k = two ? (const void*)resident_bicg_kernel<true> : (const void*)resident_bicg_kernel<false>;
-  return launch_resident(k, sm, nact, limit, args);
+bool launch_resident_bicg(hipStream_t sm, int nact, bool two, int* limits, ResidentBicg& args) {
+  const void* const k[2] = {
+      two ? (const void*)resident_bicg_kernel<true, false> : (const void*)resident_bicg_kernel<false, false>,
+      two ? nullptr : (const void*)resident_bicg_kernel<false, true>};
+  return launch_resident(k, sm, nact, limits, args);
 }
 
 template <class T>
-bool launch_resident_cg(hipStream_t sm, int nact, int* limit, ResidentCg<T>& args) {
-  return launch_resident((const void*)resident_cg_kernel<T>, sm, nact, limit, args);
+bool launch_resident_cg(hipStream_t sm, int nact, int* limits, ResidentCg<T>& args) {
+  const void* const k[2] = {(const void*)resident_cg_kernel<T, false>, (const void*)resident_cg_kernel<T, true>};
+  return launch_resident(k, sm, nact, limits, args);
 }
 template <class T>
-bool launch_resident_relax(hipStream_t sm, int nact, int mode, int* limit, ResidentRelax<T>& args) {
-  const void* k = mode == 1 ? (const void*)resident_relax_kernel<T, 1> : (const void*)resident_relax_kernel<T, 0>;
-  return launch_resident(k, sm, nact, limit, args);
+bool launch_resident_relax(hipStream_t sm, int nact, int mode, int* limits, ResidentRelax<T>& args) {
+  const void* pair = (const void*)resident_relax_kernel<T, 1, true>;
+  if (mode == 0) {  // FP64: its 36 spilled registers leave 0.95-1.15x of one launch per stage
+    pair = nullptr;
+    if constexpr (sizeof(T) == 4) pair = (const void*)resident_relax_kernel<T, 0, true>;
+  }
+  const void* one = (const void*)resident_relax_kernel<T, 1, false>;
+  if (mode == 0) one = (const void*)resident_relax_kernel<T, 0, false>;
+  const void* const k[2] = {one, pair};
+  return launch_resident(k, sm, nact, limits, args);
 }
 template bool launch_resident_cg<double>(hipStream_t, int, int*, ResidentCg<double>&);
 template bool launch_resident_cg<float>(hipStream_t, int, int*, ResidentCg<float>&);
@@ -1126,7 +1240,8 @@ template bool launch_resident_relax<float>(hipStream_t, int, int, int*, Resident
 
 void launch_unset_words(hipStream_t sm, const int* active, int nact, unsigned long long* words, size_t nslots) {
   if (nact)
-    hipLaunchKernelGGL(unset_words_kernel, dim3((RS_WORDS * nact + 255) / 256), dim3(256), 0, sm, active, nact, words, nslots);
+    hipLaunchKernelGGL(unset_words_kernel, dim3((RS_WORDS * nact + 255) / 256), dim3(256), 0, sm, active, nact, words,
+                       nslots);
 }
 
 }  // namespace ffvhc

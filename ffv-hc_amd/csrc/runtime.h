@@ -160,7 +160,7 @@ struct ffvhc_ctx {
   // resident solvers: their words (RS_WORDS per slot), how many workgroups of each kernel the device holds
   // (-1: not asked yet), and whether they are used (off after a wait in one ended without everyone)
   unsigned long long* dwords = nullptr;
-  int resident_limit[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
+  int resident_limit[16] = {-1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1};
   bool resident = true;
   // shadow residual of the compact-record methods: r0 = r (default, the reference's choice) or the
   // seeded hash vector (FFVHC_OPTION_SHADOW 1: on the 1,128-block Poisson benchmark 2-4 fewer iterations for methods 24-27 and no

@@ -102,14 +102,16 @@ int class_rows(ffvhc_ctx* c, const Coef7<T>& K, int turns, ClassRows<T>* R) {
 constexpr int kResidentTurns = 2048;
 
 enum Resident { NOT_RESIDENT, RESIDENT_DONE, RESIDENT_FAILED };
-enum { RL_BICG = 0, RL_CG = 2, RL_RELAX = 4 };  // kernels in ffvhc_ctx::resident_limit
+enum { RL_BICG = 0, RL_CG = 4, RL_RELAX = 8 };  // pairs of kernels in ffvhc_ctx::resident_limit
 
-// Whether the resident kernels (kernels_resident.hip) may run the active blocks, their words made.  The
-// line lies at one block per compute unit: below it resident solves were faster at every size tried, from
-// 1 to 256 blocks (two-level BiCGSTAB 1.4-1.6x, Jacobi BiCGSTAB 1.8-2.2x, PCG 2.4-3.6x, RBGS and
-// Jacobi 1.3-1.8x against one launch per stage); above it the blocks' vectors no longer fit on the chip.
-bool resident_ready(ffvhc_ctx* c) {
-  if (!c->resident || c->nactive < 1 || c->nactive > RS_MAX) return false;
+// Whether the resident kernels (kernels_resident.hip) may run the active blocks, at most `most`, their
+// words made.  One block per compute unit (RS_MAX): resident solves were faster at every size tried, from
+// 1 to 256 blocks (two-level BiCGSTAB 1.4-1.7x, Jacobi BiCGSTAB 1.8-2.4x, PCG 2.3-3.6x, RBGS and
+// Jacobi 1.3-2.0x against one launch per stage).  Two (RS_MAX2), where a kernel has that form: Jacobi
+// BiCGSTAB 1.7-2.1x, PCG 1.7-1.9x, Jacobi 1.0-1.3x from 257 to 512 blocks.  Above, the blocks' vectors do
+// not fit on the chip.
+bool resident_ready(ffvhc_ctx* c, int most) {
+  if (!c->resident || c->nactive < 1 || c->nactive > most) return false;
   if (!c->dwords &&
       hipMalloc(&c->dwords, sizeof(unsigned long long) * RS_WORDS * (size_t)c->cap) != hipSuccess) {
     (void)hipGetLastError();
@@ -160,7 +162,7 @@ int rbgs_core(ffvhc_ctx* c, int xf, Coef7<T> K, const T* bv, int bcg, double ome
   T* hs[2] = {(T*)X.h[0], (T*)X.h[1]};
   int n = 1, batch = kBatchMin;
   bool done = false;
-  if (mode < 2 && R.uni && resident_ready(c)) {
+  if (mode < 2 && R.uni && resident_ready(c, RS_MAX2)) {
     ResidentRelax<T> a{};
     a.active = c->dactive;
     a.blk = c->dblk;
@@ -176,7 +178,7 @@ int rbgs_core(ffvhc_ctx* c, int xf, Coef7<T> K, const T* bv, int bcg, double ome
     a.words = c->dwords;
     a.nslots = (size_t)c->cap;
     a.turns = kResidentTurns;
-    int* limit = &c->resident_limit[RL_RELAX + 2 * mode + (sizeof(T) == 4)];
+    int* limit = &c->resident_limit[RL_RELAX + 4 * mode + 2 * (sizeof(T) == 4)];
     int rc = 0;
     const Resident where = resident_run(
         c, st, hst, ids, [&] { return launch_resident_relax<T>(c->sm, c->nactive, mode, limit, a); }, &rc);
@@ -234,7 +236,7 @@ int cg_core(ffvhc_ctx* c, int xf, Coef7<T> K, const T* bv, int bcg, double omega
   fin(c, st, FIN_CG_INIT, 0);
   int n = 1, batch = kBatchMin;
   bool done = false;
-  if (R.uni && resident_ready(c)) {
+  if (R.uni && resident_ready(c, RS_MAX2)) {
     ResidentCg<T> a{};
     a.active = c->dactive;
     a.blk = c->dblk;
@@ -251,7 +253,7 @@ int cg_core(ffvhc_ctx* c, int xf, Coef7<T> K, const T* bv, int bcg, double omega
     a.turns = kResidentTurns;
     const Resident where = resident_run(
         c, st, hst, ids,
-        [&] { return launch_resident_cg<T>(c->sm, c->nactive, &c->resident_limit[RL_CG + (sizeof(T) == 4)], a); }, &rc);
+        [&] { return launch_resident_cg<T>(c->sm, c->nactive, &c->resident_limit[RL_CG + 2 * (sizeof(T) == 4)], a); }, &rc);
     if (rc) return rc;
     if (where == RESIDENT_FAILED)  // again from the x there is (a starting guess like any other)
       return cg_core<T>(c, xf, K, bv, bcg, omega, countMax, eps, st, hst, outer, launched);
@@ -311,7 +313,7 @@ Resident bicgstab_resident(ffvhc_ctx* c, T* x, const Coef7<T>& K, const BiVecs<T
   } else {
     const bool two = o.gs == BiOpts::GSC && o.cinv && o.mult && !o.hash_r0 && o.trec;
     const bool jacobi = o.gs == BiOpts::NONE && !o.A32 && R.uni;
-    if (c->graphs || !(two || jacobi) || !resident_ready(c)) return NOT_RESIDENT;
+    if (c->graphs || !(two || jacobi) || !resident_ready(c, two ? RS_MAX : RS_MAX2)) return NOT_RESIDENT;
     ResidentBicg a{};
     a.active = c->dactive;
     a.blk = c->dblk;
@@ -339,7 +341,7 @@ Resident bicgstab_resident(ffvhc_ctx* c, T* x, const Coef7<T>& K, const BiVecs<T
     a.turns = kResidentTurns;
     return resident_run(
         c, st, hst, ids,
-        [&] { return launch_resident_bicg(c->sm, c->nactive, two, &c->resident_limit[RL_BICG + two], a); }, rc);
+        [&] { return launch_resident_bicg(c->sm, c->nactive, two, &c->resident_limit[RL_BICG + 2 * two], a); }, rc);
   }
 }
 

@@ -322,8 +322,9 @@ class Context:
         check(_L.ffvhc_ctx_set_option(self.h, 6, int(bool(on))), "ffvhc_ctx_set_option")
 
     def set_resident(self, on):
-        """Run solves of at most 256 active blocks in one launch whose blocks stay on the chip (default), or
-        launch every stage of every iteration."""
+        """Run solves of at most 256 active blocks (512 for BiCGSTAB, PCG, Jacobi and FP32 RBGS on the matrix
+        itself) in one launch whose blocks stay on the chip (default), or launch every stage of every
+        iteration."""
         check(_L.ffvhc_ctx_set_option(self.h, 7, int(bool(on))), "ffvhc_ctx_set_option")
 
     def set_classes(self, on):

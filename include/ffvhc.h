@@ -129,9 +129,10 @@ long long ffvhc_ctx_device_bytes(const ffvhc_ctx* ctx);
  * first coarse application instead of a launch of its own, except after the last iteration of a
  * launch batch; 0 launches it every iteration.  The results are identical. */
 #define FFVHC_OPTION_FUSE_FIN 6
-/* FFVHC_OPTION_RESIDENT: 1 (default) lets solves of at most 256 active blocks (on a device that holds
- * as many workgroups at once) run in one launch, each block's vectors staying on the chip; 0 launches
- * every stage of every iteration.  The results are identical. */
+/* FFVHC_OPTION_RESIDENT: 1 (default) lets solves of at most 256 active blocks (512 for BiCGSTAB, PCG,
+ * Jacobi and FP32 RBGS on the matrix itself; on a device that holds as many workgroups at once) run in
+ * one launch, each block's vectors staying on the chip; 0 launches every stage of every iteration.  The
+ * results are identical. */
 #define FFVHC_OPTION_RESIDENT 7
 int ffvhc_ctx_set_option(ffvhc_ctx* ctx, int option, int value);
 
