@@ -131,7 +131,7 @@ int ensure_second_buffer(ffvhc_ctx* ctx, int field) {
   return 0;
 }
 
-int upload_case_meta(ffvhc_ctx* c, int id) {
+static void make_case_meta(ffvhc_ctx* c, int id) {
   const CaseRec& r = c->cases[id];
   DevCase& d = c->hcase[id];
   d.slot_begin = r.slot_begin;
@@ -157,7 +157,26 @@ int upload_case_meta(ffvhc_ctx* c, int id) {
   // Solver.cpp:3347-3355: the X_M inflow value of UX ramps up over the acceleration steps
   if (r.accel_steps > 0 && r.step <= r.accel_steps)
     d.bcv[BC_UX][0] = r.params.bcv[BC_UX][0] * (double)r.step / (double)r.accel_steps;
-  HIPCHK(hipMemcpyAsync(c->dcase + id, &d, sizeof(DevCase), hipMemcpyHostToDevice, c->sm));
+  c->pcase[id] = d;
+}
+
+// One copy per run of consecutive ids, in selection order; the entries are read from pinned memory while the
+// stream runs, so a caller that does not wait before it returns must not be followed by another change.
+int send_case_meta(ffvhc_ctx* c, const std::vector<int>& ids) {
+  for (size_t i = 0; i < ids.size();) {
+    size_t e = i;
+    do make_case_meta(c, ids[e++]);
+    while (e < ids.size() && ids[e] == ids[e - 1] + 1);
+    HIPCHK(hipMemcpyAsync(c->dcase + ids[i], c->pcase.data() + ids[i], sizeof(DevCase) * (e - i), hipMemcpyHostToDevice,
+                          c->sm));
+    i = e;
+  }
+  return 0;
+}
+
+int upload_case_meta(ffvhc_ctx* c, int id) {
+  int rc = send_case_meta(c, {id});
+  if (rc) return rc;
   HIPCHK(hipStreamSynchronize(c->sm));
   return 0;
 }
@@ -279,6 +298,10 @@ int ffvhc_ctx_create(int device, long long max_blocks, ffvhc_ctx** out) {
   c->hst.assign(MAX_CASES, SolveState{});
   c->hst2.assign(MAX_CASES, SolveState{});
   c->fields.reserve(MAX_FIELDS);
+  HIPCHK(c->pcase.reserve(MAX_CASES));
+  HIPCHK(c->pst.reserve(MAX_CASES));
+  HIPCHK(c->presult.reserve(5 * (size_t)MAX_CASES));
+  for (auto& e : c->ev_step) HIPCHK(hipEventCreate(&e));
   HIPCHK(hipMalloc(&c->dblk, sizeof(DevBlock) * max_blocks));
   HIPCHK(hipMalloc(&c->dcase, sizeof(DevCase) * MAX_CASES));
   HIPCHK(hipMalloc(&c->dactive, sizeof(int) * max_blocks));
@@ -336,6 +359,7 @@ void ffvhc_ctx_destroy(ffvhc_ctx* c) {
   (void)hipFree(c->dflag);
   (void)hipFree(c->dcid);
   if (c->blas) (void)rocblas_destroy_handle((rocblas_handle)c->blas);
+  for (auto& e : c->ev_step) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(c->sm);
   if (c->sc) {
     (void)hipEventDestroy(c->ev_cs);

@@ -37,6 +37,31 @@ struct FieldRec {
   void* h[2] = {nullptr, nullptr};  // halo, ping-pong
 };
 
+// Page-locked host memory.  What a call reads back is copied or written there: a copy to pageable memory
+// goes through the runtime's staging buffer and waits for itself.
+template <class T>
+struct Pinned {
+  T* p = nullptr;
+  size_t n = 0;
+  Pinned() = default;
+  Pinned(const Pinned&) = delete;
+  Pinned& operator=(const Pinned&) = delete;
+  ~Pinned() {
+    if (p) (void)hipHostFree(p);
+  }
+  hipError_t reserve(size_t count) {  // at least `count` entries; the old ones are not kept
+    if (count <= n) return hipSuccess;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+    const hipError_t e = hipHostMalloc((void**)&p, count * sizeof(T), hipHostMallocDefault);
+    if (e == hipSuccess) n = count;
+    return e;
+  }
+  T* data() const { return p; }
+  T& operator[](size_t i) const { return p[i]; }
+};
+
 struct CaseRec {
   bool used = false;
   int slot_begin = 0;
@@ -59,6 +84,10 @@ struct ffvhc_ctx {
   std::vector<ffvhc::DevBlock> hblk;
   ffvhc::DevBlock* dblk = nullptr;
   std::vector<ffvhc::DevCase> hcase;
+  ffvhc::Pinned<ffvhc::DevCase> pcase;       // hcase as last sent to dcase
+  ffvhc::Pinned<ffvhc::SolveState> pst;      // where the states of a solve are read back
+  ffvhc::Pinned<double> presult;             // where kernels write per-case results
+  hipEvent_t ev_step[4] = {};                // the stages of ffvhc_step
   ffvhc::DevCase* dcase = nullptr;
   std::vector<ffvhc::CaseRec> cases;
   // geometry per slot: cut distances (float, exact: Cutlib stores float32), cell flags
@@ -104,9 +133,9 @@ struct ffvhc_ctx {
   int coarse_gemm_min = 2048;
   // host copies the setups read back or upload asynchronously; they live here so that they
   // outlive the copies (a setup returns without waiting for its last kernels)
-  std::vector<double> hcrows;   // 25 coarse row entries per slot
+  ffvhc::Pinned<double> hcrows;  // 25 coarse row entries per slot
   std::vector<long long> hcoff;  // the offsets uploaded to dcoff
-  std::vector<int> hcuni;        // class-uniform flag per slot
+  ffvhc::Pinned<int> hcuni;      // class-uniform flag per slot
   // the coarse inversion runs on stream sc (default priority) beside the solver's first kernels
   // on sm: ev_cs orders it after the assembly on sm, ev_cd marks its end; coarse_pending says
   // that sm has not yet been made to wait for ev_cd
@@ -183,5 +212,6 @@ int alloc_field(ffvhc_ctx* ctx, int prec, int* field);
 int scratch_field(ffvhc_ctx* ctx, int prec, int role, int* field);
 bool field_ok(ffvhc_ctx* ctx, int f, int prec);
 int upload_case_meta(ffvhc_ctx* c, int id);
+int send_case_meta(ffvhc_ctx* c, const std::vector<int>& ids);  // without waiting
 int host_impose_bc(ffvhc_ctx* c, int id, double* padded, int g, int bcg, int updater);
 }  // namespace ffvhc

@@ -48,10 +48,18 @@ Coef7<T> coef(ffvhc_ctx* c, const int* A) {
   return k;
 }
 
+int sync_state(ffvhc_ctx* c, SolveState* dst, std::vector<SolveState>& hst) {
+  const size_t n = c->cases.size();
+  HIPCHK(hipMemcpyAsync(c->pst.data(), dst, sizeof(SolveState) * n, hipMemcpyDeviceToHost, c->sm));
+  HIPCHK(hipStreamSynchronize(c->sm));
+  std::copy(c->pst.data(), c->pst.data() + n, hst.begin());
+  return 0;
+}
+
 int read_state(ffvhc_ctx* c, SolveState* dst, std::vector<SolveState>& hst, const std::vector<int>& ids,
                bool* all_done) {
-  HIPCHK(hipMemcpyAsync(hst.data(), dst, sizeof(SolveState) * c->cases.size(), hipMemcpyDeviceToHost, c->sm));
-  HIPCHK(hipStreamSynchronize(c->sm));
+  int rc = sync_state(c, dst, hst);
+  if (rc) return rc;
   *all_done = true;
   for (int id : ids)
     if (!hst[id].done) *all_done = false;
@@ -453,12 +461,6 @@ int report(ffvhc_ctx* c, const std::vector<SolveState>& hst, int* count, double*
   return status;
 }
 
-int sync_state(ffvhc_ctx* c, SolveState* dst, std::vector<SolveState>& hst) {
-  HIPCHK(hipStreamSynchronize(c->sm));
-  HIPCHK(hipMemcpy(hst.data(), dst, sizeof(SolveState) * c->cases.size(), hipMemcpyDeviceToHost));
-  return 0;
-}
-
 template <class T>
 int rbgs_fixed_run(ffvhc_ctx* c, int x, const int* A, int b, int bcg, double omega, int nsweep, double* ms) {
   int rc = ensure_second_buffer(c, x);
@@ -686,9 +688,8 @@ int coarse_rows_launch(ffvhc_ctx* c, const Coef7<double>& K) {
   double* drows = (double*)c->fields[fr].d[0];  // 25 doubles per slot (cap * NC doubles available)
   launch_coarse_rows(c->sm, c->dactive, c->nactive, c->dblk, K, drows);
   HIPCHK(hipGetLastError());
-  c->hcrows.resize((size_t)c->cap * 25);
-  HIPCHK(hipMemcpyAsync(c->hcrows.data(), drows, c->hcrows.size() * sizeof(double), hipMemcpyDeviceToHost,
-                        c->sm));
+  HIPCHK(c->hcrows.reserve((size_t)c->cap * 25));
+  HIPCHK(hipMemcpyAsync(c->hcrows.data(), drows, (size_t)c->cap * 25 * sizeof(double), hipMemcpyDeviceToHost, c->sm));
   return 0;
 }
 
@@ -710,7 +711,7 @@ int coarse_finish(ffvhc_ctx* c, BiOpts* o, double* ac_out, double* inv_out) {
     HIPCHK(hipEventCreateWithFlags(&c->ev_cd, hipEventDisableTiming));
   }
   const double* drows = (const double*)c->fields[fr].d[0];
-  const std::vector<double>& rows = c->hcrows;
+  const double* const rows = c->hcrows.data();
   const std::vector<int> ids = selected_cases(c);
   // FP64 operators / inverses at off[case] (n x n); their FP32 copies at offp[case] with the row
   // pitch padded to a multiple of 4 (float4 rows)
@@ -834,7 +835,7 @@ int class_launch(ffvhc_ctx* c, const Coef7<double>& K) {
   launch_stencil_classes(c->sm, c->dactive, c->nactive, K, c->dcuni, c->dctab, c->dcex,
                          (uint4*)c->dctrec);
   HIPCHK(hipGetLastError());
-  c->hcuni.resize(cap);
+  HIPCHK(c->hcuni.reserve(cap));
   HIPCHK(hipMemcpyAsync(c->hcuni.data(), c->dcuni, cap * sizeof(int), hipMemcpyDeviceToHost, c->sm));
   return 0;
 }
@@ -1635,13 +1636,12 @@ template <class Launch>
 static int case_triples(ffvhc_ctx* c, double* f, Launch launch) {
   int rc = refresh_active(c);
   if (rc) return rc;
-  double* dout = nullptr;
-  HIPCHK(hipMallocAsync((void**)&dout, sizeof(double) * 3 * std::max(c->ncaseact, 1), c->sm));
-  launch(dout);
+  // the kernel writes the triples to the host (a device buffer and a copy back took 12 us more)
+  const double* const h = c->presult.data();
+  void* dout = nullptr;
+  HIPCHK(hipHostGetDevicePointer(&dout, c->presult.data(), 0));
+  launch((double*)dout);
   HIPCHK(hipGetLastError());
-  std::vector<double> h(3 * std::max(c->ncaseact, 1), 0.0);
-  HIPCHK(hipMemcpyAsync(h.data(), dout, sizeof(double) * 3 * c->ncaseact, hipMemcpyDeviceToHost, c->sm));
-  HIPCHK(hipFreeAsync(dout, c->sm));
   HIPCHK(hipStreamSynchronize(c->sm));
   // caseact lists the selected cases with blocks in selection order
   const std::vector<int> ids = selected_cases(c);
@@ -1732,15 +1732,12 @@ int ffvhc_field_stats(ffvhc_ctx* c, int f, double* out) {
   int rc = refresh_active(c);
   if (rc) return rc;
   const std::vector<int> ids = selected_cases(c);
-  const int n = std::max(c->ncaseact, 1);
-  double* dout = nullptr;
-  HIPCHK(hipMallocAsync((void**)&dout, sizeof(double) * 5 * n, c->sm));
+  const double* const h = c->presult.data();
+  void* dout = nullptr;
+  HIPCHK(hipHostGetDevicePointer(&dout, c->presult.data(), 0));
   launch_stats(c->sm, c->dactive, c->nactive, c->dcaseact, c->ncaseact, c->dcase, (const double*)c->fields[f].d[0],
-               c->dpart, (size_t)c->cap, dout);
+               c->dpart, (size_t)c->cap, (double*)dout);
   HIPCHK(hipGetLastError());
-  std::vector<double> h(5 * n, 0.0);
-  HIPCHK(hipMemcpyAsync(h.data(), dout, sizeof(double) * 5 * c->ncaseact, hipMemcpyDeviceToHost, c->sm));
-  HIPCHK(hipFreeAsync(dout, c->sm));
   HIPCHK(hipStreamSynchronize(c->sm));
   size_t q = 0;
   for (size_t i = 0; i < ids.size(); i++) {
@@ -1803,10 +1800,8 @@ int ffvhc_step(ffvhc_ctx* c, ffvhc_step_fields* F, const ffvhc_step_params* P, f
   int rc = refresh_active(c);
   if (rc) return rc;
   const std::vector<int> ids = selected_cases(c);
-  for (int id : ids) {
-    rc = upload_case_meta(c, id);
-    if (rc) return rc;
-  }
+  rc = send_case_meta(c, ids);
+  if (rc) return rc;
   auto D = [&](int f) { return (double*)c->fields[f].d[0]; };
   auto H = [&](int f) { return (double*)c->fields[f].h[0]; };
   StepFields S;
@@ -1837,8 +1832,7 @@ int ffvhc_step(ffvhc_ctx* c, ffvhc_step_fields* F, const ffvhc_step_params* P, f
     }
     launch_ghost_pull<double>(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, G, c->multilevel);
   };
-  hipEvent_t ev[4];
-  for (auto& e : ev) HIPCHK(hipEventCreate(&e));
+  hipEvent_t(&ev)[4] = c->ev_step;
   HIPCHK(hipEventRecord(ev[0], c->sm));
   const size_t nc = ids.size();
   std::vector<int> cntu(3 * nc, 0);
@@ -1922,7 +1916,6 @@ int ffvhc_step(ffvhc_ctx* c, ffvhc_step_fields* F, const ffvhc_step_params* P, f
   HIPCHK(hipEventElapsedTime(&t01, ev[0], ev[1]));
   HIPCHK(hipEventElapsedTime(&t12, ev[1], ev[2]));
   HIPCHK(hipEventElapsedTime(&t23, ev[2], ev[3]));
-  for (auto& e : ev) (void)hipEventDestroy(e);
   if (stage_ms) {
     stage_ms[0] = t01 + t12 + t23;
     stage_ms[1] = 0.0;

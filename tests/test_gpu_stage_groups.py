@@ -45,3 +45,34 @@ def test_stats_of_many_blocks(where):
         assert list(got[1:]) == [2.0, -3.0, 3.0, 1e-9]
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("ids", [[2, 0], [0, 1, 3], [3, 2, 1, 0]])
+def test_parameters_of_selected_cases(ids):
+    """Each selected case steps with its own dt, whatever runs of ids the selection makes."""
+    tree = ffvhc.Tree(root=(2, 1, 1), root_length=1.0)
+    ctx = ffvhc.Context(max_blocks=4 * tree.nblk)
+    try:
+        F = ctx.step_fields()
+        rng = np.random.default_rng(8)
+        start = {f: rng.standard_normal((tree.nblk,) + (N + 2 * G,) * 3) for f in (F.ux, F.uy, F.uz)}
+        cids = [ctx.add_case(tree, ffvhc.case_params(mu=0.01, dt=0.001 * (1 + q), bc=BC)) for q in range(4)]
+
+        def go(sel):
+            for q in sel:
+                for f in (F.p, F.lapp, *F.v, *F.uc, *F.ucp, *F.ud, *F.udp):
+                    ctx.upload(f, cids[q], np.zeros_like(start[F.ux]))
+                for f, x in start.items():
+                    ctx.upload(f, cids[q], x)
+                ctx.set_step(cids[q], 0, 0)
+            ctx.select([cids[q] for q in sel])
+            _, _, rc = ctx.step(F, solver=0, omega=1.2, count_max=3, eps=0.0, ncases=len(sel))
+            assert rc == 0
+            return {q: ctx.download(F.ux, cids[q]) for q in sel}
+
+        together = go(ids)
+        for q in ids:
+            assert np.array_equal(together[q], go([q])[q])
+        assert len({together[q].tobytes() for q in ids}) == len(ids)
+    finally:
+        ctx.close()
