@@ -151,6 +151,13 @@ __device__ inline int thread_here() {
   return t;
 }
 
+// a or b by value: the conditional operator on two array elements selects an address, which would put
+// the arrays in memory
+template <class T>
+__device__ inline T pick(bool c, T a, T b) {
+  return c ? a : b;
+}
+
 // f(true_type) for a class-uniform block, f(false_type) else (uniform over the workgroup)
 template <class T, class F>
 __device__ inline void by_class(const ClassRows<T>& R, int slot, const F& f) {

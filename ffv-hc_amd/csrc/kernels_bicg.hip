@@ -397,7 +397,7 @@ template void launch_class_rows<float>(hipStream_t, const int*, int, Coef7<float
 // z <- z + omega (u - sum_q w_q z_q - z).  The block's z lives in LDS; each of the GSK_NT threads
 // keeps u and the couplings of half an (i, j) column (8 cells) in registers, so the sweeps after
 // the first read no HBM.  The couplings to cells outside the block are zeroed in the registers
-// (ghost values are zero in the block-local system), so a sweep reads its six LDS neighbours at
+// (ghost values are zero in the block-local system), so a sweep reads its LDS neighbours at
 // fixed offsets with no bounds test: the x / y offsets of an edge cell then wrap to a cell of
 // the same colour of another column (multiplied by zero) and the k offsets of the end planes to
 // a zero plane below and above the block.
@@ -411,18 +411,16 @@ constexpr int GSK_NK = NB * 256 / GSK_NT;  // cells of a column per thread
 // REG 1 (every block of the launch class-uniform): the records are the block's class records
 // trec[slot][27] instead of the per-cell array, and the sweeps keep one set of couplings for the
 // thread's inner cells and one for its end cell (k = 0 or NB - 1) instead of one per cell, which
-// leaves registers for three workgroups per CU.  REG 2 (mixed launch): each block takes its
-// records from the class rows when uni[slot] is set, else per cell.
+// leaves registers for three workgroups per CU.  REG 2 (mixed launch): so for the blocks with uni[slot]
+// set; the others' sweeps read the couplings again each half sweep (from L2), so that three workgroups
+// fit a CU here too.  REG 3: the same with the others' couplings per cell in registers, REG 0: so all
+// blocks'; two workgroups a CU.
 template <class T, int MODE, int NS, bool MUL, int REG>
-__global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1 ? 6 : 1))) void bi_precond_gsk_kernel(const int* __restrict__ active,
-                                                               const DevBlock* __restrict__ blk,
-                                                               const DevCase* __restrict__ cs,
-                                                               const SolveState* __restrict__ st,
-                                                               const uint4* __restrict__ rec, BiVecs<T> V,
-                                                               int count, double* __restrict__ vs_out,
-                                                               const double* __restrict__ ce,
-                                                               const uint4* __restrict__ trec,
-                                                               const int* __restrict__ uni) {
+__global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1 || REG == 2 ? 6 : 1))) void bi_precond_gsk_kernel(
+    const int* __restrict__ active, const DevBlock* __restrict__ blk, const DevCase* __restrict__ cs,
+    const SolveState* __restrict__ st, const uint4* __restrict__ rec, BiVecs<T> V, int count,
+    double* __restrict__ vs_out, const double* __restrict__ ce, const uint4* __restrict__ trec,
+    const int* __restrict__ uni) {
   __shared__ double zpad[NC + 2 * NF];  // z with a zero plane below (k = -1) and above (k = NB)
   __shared__ double red[GSK_NT / 64];
   const int slot = active[blockIdx.x];
@@ -448,32 +446,12 @@ __global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1
   // arguments); FIN_BI_XR of the previous iteration stored it in iter
   const bool first = (count > 0 ? count : st[c].iter + 1) == 1 || st[c].restart;
   const int par = (tx + ty) & 1;  // red cells of this column: k = kb + 2m + par (kb even)
-  auto zi = [](int i, int j, int k) { return i + NB * (j + NB * k); };
-  // per colour (index m: k = kb + 2m + par for red, kb + 2m + 1 - par for black), compile-time
-  // indexed so that they stay in registers
-  double ur[GSK_NK / 2], ub[GSK_NK / 2];
-  uint32_t wr[GSK_NK / 2][3], wb[GSK_NK / 2][3];
-  double vsum = 0.0;
+  double* const z0 = z + o0;
   // couplings kept for the sweeps: those to cells outside the block zeroed (per half word)
   const uint32_t mx = (tx == 0 ? 0xffff0000u : ~0u) & (tx == NB - 1 ? 0x0000ffffu : ~0u);
   const uint32_t my = (ty == 0 ? 0xffff0000u : ~0u) & (ty == NB - 1 ? 0x0000ffffu : ~0u);
-  // REG: the class records of the thread's inner cells and of its end cell (k = 0 for the lower
-  // half column, NB - 1 for the upper), and their couplings as kept for the sweeps
-  const bool cls = REG == 1 || (REG == 2 && uni[slot] != 0);  // uniform over the workgroup
-  uint4 rin = {}, rend = {};
-  uint32_t win[3] = {}, wend[3] = {};
-  if (REG != 0 && cls) {
-    const uint4* tr = trec + (size_t)slot * 27 + stencil_class1(tx) + 3 * stencil_class1(ty);
-    rin = tr[9];
-    rend = tr[kb == 0 ? 0 : 18];
-    win[0] = rin.y & mx;
-    win[1] = rin.z & my;
-    win[2] = rin.w;
-    wend[0] = rend.y & mx;
-    wend[1] = rend.z & my;
-    wend[2] = rend.w & (kb == 0 ? 0xffff0000u : 0x0000ffffu);
-  }
   const bool lower = kb == 0;
+  const bool cls = REG == 1 || (REG > 1 && uni[slot] != 0);  // uniform over the workgroup
   // MUL: e of this block (eo) and of the block the ghost value of the x, y and z face this
   // thread's cells touch comes from (ex: face x- when tx = 0, else x+; ey likewise; ez: z- for the
   // lower half column, z+ for the upper).  A half column never straddles a subface boundary, so
@@ -489,123 +467,158 @@ __global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1
     ey = ce[sy];
     ez = ce[sz];
   }
-#pragma unroll
-  for (int k0 = 0; k0 < GSK_NK; k0 += 4) {
-    T rv[4], pv[4], qv[4];
-    uint4 rc[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      const unsigned o = o0 + NF * (k0 + kk);
-      // streamed once through this kernel: non-temporal loads and stores leave the caches to what
-      // the next kernels read (measured: this kernel 3% faster, the matvecs after it 3-7%)
-      rv[kk] = __builtin_nontemporal_load(rb + o);
-      if (MODE == 1 || !first) qv[kk] = __builtin_nontemporal_load(qb + o);
-      if (MODE == 0 && !first) pv[kk] = __builtin_nontemporal_load(vb + o);
-      if (REG == 0 || (REG == 2 && !cls)) rc[kk] = recb[o];
+  // the rest in two forms, so that a class-row block's holds no per-cell couplings
+  auto rest = [&](auto cls_tag) __attribute__((always_inline)) {
+    constexpr bool CLS = decltype(cls_tag)::value, AGAIN = !CLS && REG == 2;
+    // per colour (index m: k = kb + 2m + par for red, kb + 2m + 1 - par for black), compile-time
+    // indexed so that they stay in registers
+    double ur[GSK_NK / 2], ub[GSK_NK / 2];
+    uint32_t wr[GSK_NK / 2][3], wb[GSK_NK / 2][3];  // !CLS
+    double vsum = 0.0;
+    // CLS: the class records of the thread's inner cells and of its end cell (k = 0 for the lower
+    // half column, NB - 1 for the upper), and their couplings as kept for the sweeps
+    uint4 rin = {}, rend = {};
+    uint32_t win[3] = {}, wend[3] = {};
+    if constexpr (CLS) {
+      const uint4* tr = trec + (size_t)slot * 27 + stencil_class1(tx) + 3 * stencil_class1(ty);
+      rin = tr[9];
+      rend = tr[kb == 0 ? 0 : 18];
+      win[0] = rin.y & mx;
+      win[1] = rin.z & my;
+      win[2] = rin.w;
+      wend[0] = rend.y & mx;
+      wend[1] = rend.z & my;
+      wend[2] = rend.w & (kb == 0 ? 0xffff0000u : 0x0000ffffu);
     }
+    constexpr int KB = AGAIN ? 2 : 4;  // cells loaded at a time
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      const int k = k0 + kk;  // relative to kb
-      if (REG != 0 && cls) {  // the end cell of the half column is k = 0 (lower) or GSK_NK - 1 (upper)
-        if (k == 0) rc[kk] = lower ? rend : rin;
-        else if (k == GSK_NK - 1) rc[kk] = lower ? rin : rend;
-        else rc[kk] = rin;
+    for (int k0 = 0; k0 < GSK_NK; k0 += KB) {
+      T rv[KB], pv[KB], qv[KB];
+      uint4 rc[KB];
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++) {
+        const unsigned o = o0 + NF * (k0 + kk);
+        // streamed once through this kernel: non-temporal loads and stores leave the caches to what
+        // the next kernels read (measured: this kernel 3% faster, the matvecs after it 3-7%)
+        rv[kk] = __builtin_nontemporal_load(rb + o);
+        if (MODE == 1 || !first) qv[kk] = __builtin_nontemporal_load(qb + o);
+        if (MODE == 0 && !first) pv[kk] = __builtin_nontemporal_load(vb + o);
+        if constexpr (!CLS) rc[kk] = recb[o];
       }
-      // FP64 vectors: the recurrence's own values; FP32 vectors (an inner solve of a defect
-      // correction): formed in FP64 and rounded once when stored
-      double v;
-      if (MODE == 0)
-        v = first ? (double)rv[kk] : (double)rv[kk] + beta * ((double)pv[kk] + ng * (double)qv[kk]);
-      else
-        v = na * (double)qv[kk] + (double)rv[kk];
-      if constexpr (sizeof(T) == 4) v = (double)(T)v;  // the value the recurrence keeps
-      __builtin_nontemporal_store((T)v, vb + o0 + NF * k);
-      vsum += v;
-      double uk = v * (double)__uint_as_float(rc[kk].x);
-      const int ka = kb + k;
-      if constexpr (MUL) {
-        uk -= eo + half_lo(rc[kk].y) * (tx > 0 ? eo : ex) + half_hi(rc[kk].y) * (tx < NB - 1 ? eo : ex) +
-              half_lo(rc[kk].z) * (ty > 0 ? eo : ey) + half_hi(rc[kk].z) * (ty < NB - 1 ? eo : ey) +
-              half_lo(rc[kk].w) * (ka > 0 ? eo : ez) + half_hi(rc[kk].w) * (ka < NB - 1 ? eo : ez);
-      }
-      const int m = k >> 1;
-      const uint32_t mz = (ka == 0 ? 0xffff0000u : ~0u) & (ka == NB - 1 ? 0x0000ffffu : ~0u);
-      if ((k & 1) == par) {
-        ur[m] = uk;
-        if constexpr (REG != 1) {
-          wr[m][0] = rc[kk].y & mx;
-          wr[m][1] = rc[kk].z & my;
-          wr[m][2] = rc[kk].w & mz;
-        }
-      } else {
-        ub[m] = uk;
-        if constexpr (REG != 1) {
-          wb[m][0] = rc[kk].y & mx;
-          wb[m][1] = rc[kk].z & my;
-          wb[m][2] = rc[kk].w & mz;
+      if constexpr (CLS) {  // the end cell of the half column is k = 0 (lower) or GSK_NK - 1 (upper)
+#pragma unroll
+        for (int kk = 0; kk < KB; kk++) {
+          const int k = k0 + kk;
+          rc[kk] = k == 0 ? pick(lower, rend, rin) : k == GSK_NK - 1 ? pick(lower, rin, rend) : rin;
         }
       }
-    }
-  }
-  if (vs_out) {
-    const double sv = block_sum<GSK_NT>(vsum, red);
-    if (t == 0) vs_out[slot] = sv;
-  }
-  // first red half sweep: every neighbour is still zero; the black cells start at zero (the
-  // wrapped reads of the first black half sweep must see finite values)
 #pragma unroll
-  for (int m = 0; m < GSK_NK / 2; m++) {
-    z[zi(tx, ty, kb + 2 * m + par)] = omega * ur[m];
-    z[zi(tx, ty, kb + 2 * m + 1 - par)] = 0.0;
-  }
-  __syncthreads();
-  // one half sweep over this column's cells of one colour; from_zero: the cells' old values are
-  // zero (first visit)
-  auto half = [&](auto red_tag, bool from_zero) {
-    constexpr bool RED = decltype(red_tag)::value;
-    const int cp = RED ? par : 1 - par;  // this colour's cells: k = kb + 2m + cp
-    const int kp = kb + cp;
+      for (int kk = 0; kk < KB; kk++) {
+        const int k = k0 + kk;  // relative to kb
+        // FP64 vectors: the recurrence's own values; FP32 vectors (an inner solve of a defect
+        // correction): formed in FP64 and rounded once when stored
+        double v;
+        if (MODE == 0)
+          v = first ? (double)rv[kk] : (double)rv[kk] + beta * ((double)pv[kk] + ng * (double)qv[kk]);
+        else
+          v = na * (double)qv[kk] + (double)rv[kk];
+        if constexpr (sizeof(T) == 4) v = (double)(T)v;  // the value the recurrence keeps
+        __builtin_nontemporal_store((T)v, vb + o0 + NF * k);
+        vsum += v;
+        double uk = v * (double)__uint_as_float(rc[kk].x);
+        const int ka = kb + k;
+        if constexpr (MUL) {
+          uk -= eo + half_lo(rc[kk].y) * (tx > 0 ? eo : ex) + half_hi(rc[kk].y) * (tx < NB - 1 ? eo : ex) +
+                half_lo(rc[kk].z) * (ty > 0 ? eo : ey) + half_hi(rc[kk].z) * (ty < NB - 1 ? eo : ey) +
+                half_lo(rc[kk].w) * (ka > 0 ? eo : ez) + half_hi(rc[kk].w) * (ka < NB - 1 ? eo : ez);
+        }
+        const int m = k >> 1;
+        const uint32_t mz = (ka == 0 ? 0xffff0000u : ~0u) & (ka == NB - 1 ? 0x0000ffffu : ~0u);
+        if ((k & 1) == par) {
+          ur[m] = uk;
+          if constexpr (!CLS && !AGAIN) {
+            wr[m][0] = rc[kk].y & mx;
+            wr[m][1] = rc[kk].z & my;
+            wr[m][2] = rc[kk].w & mz;
+          }
+        } else {
+          ub[m] = uk;
+          if constexpr (!CLS && !AGAIN) {
+            wb[m][0] = rc[kk].y & mx;
+            wb[m][1] = rc[kk].z & my;
+            wb[m][2] = rc[kk].w & mz;
+          }
+        }
+      }
+    }
+    if (vs_out) {
+      const double sv = block_sum<GSK_NT>(vsum, red);
+      if (t == 0) vs_out[slot] = sv;
+    }
+    // first red half sweep: every neighbour is still zero; the black cells start at zero (the
+    // wrapped reads of the first black half sweep must see finite values)
 #pragma unroll
     for (int m = 0; m < GSK_NK / 2; m++) {
-      const int k = 2 * m + kp;
-      uint32_t w[3];
-      if constexpr (REG == 1) {
-        // the end cell: m = 0 with cp = 0 (lower half), m = last with cp = 1 (upper half)
-        const bool end = m == 0 ? (lower && cp == 0) : m == GSK_NK / 2 - 1 ? (!lower && cp == 1) : false;
-#pragma unroll
-        for (int b = 0; b < 3; b++) w[b] = end ? wend[b] : win[b];
-      } else {
-#pragma unroll
-        for (int b = 0; b < 3; b++) w[b] = RED ? wr[m][b] : wb[m][b];
-      }
-      // keep the couplings packed across sweeps (an empty asm hides that the unpacked values
-      // of the last sweep could be reused, which would cost 12 more registers per cell)
-      asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]));
-      const double* zc = z + zi(tx, ty, k);
-      double sum = half_lo(w[0]) * zc[-1];
-      sum = __builtin_fma(half_hi(w[0]), zc[1], sum);
-      sum = __builtin_fma(half_lo(w[1]), zc[-NB], sum);
-      sum = __builtin_fma(half_hi(w[1]), zc[NB], sum);
-      sum = __builtin_fma(half_lo(w[2]), zc[-NB * NB], sum);
-      sum = __builtin_fma(half_hi(w[2]), zc[NB * NB], sum);
-      const double zn = (RED ? ur[m] : ub[m]) - sum;
-      if (from_zero) {
-        z[zi(tx, ty, k)] = omega * zn;
-      } else {
-        const double zo = z[zi(tx, ty, k)];
-        z[zi(tx, ty, k)] = __builtin_fma(omega, zn - zo, zo);
-      }
+      z0[NF * (2 * m + par)] = omega * ur[m];
+      z0[NF * (2 * m + 1 - par)] = 0.0;
     }
     __syncthreads();
-  };
-  using Red = std::true_type;
-  using Black = std::false_type;
-  half(Black{}, true);
+    // one half sweep over this column's cells of one colour; from_zero: the cells' old values are
+    // zero (first visit)
+    auto half = [&](auto red_tag, bool from_zero) __attribute__((always_inline)) {
+      constexpr bool RED = decltype(red_tag)::value;
+      const int cp = RED ? par : 1 - par;  // this colour's cells: k = kb + 2m + cp
 #pragma unroll
-  for (int sweep = 1; sweep < NS; sweep++) {
-    half(Red{}, false);
-    half(Black{}, false);
-  }
+      for (int m = 0; m < GSK_NK / 2; m++) {
+        uint32_t w[3];
+        if constexpr (CLS) {
+          // the end cell: m = 0 with cp = 0 (lower half), m = last with cp = 1 (upper half)
+          const bool end = m == 0 ? (lower && cp == 0) : m == GSK_NK / 2 - 1 ? (!lower && cp == 1) : false;
+#pragma unroll
+          for (int b = 0; b < 3; b++) w[b] = end ? wend[b] : win[b];
+        } else if constexpr (AGAIN) {
+          const int u = thread_here(), i = u & 15, j = (u >> 4) & 15, k = (u >> 8) * GSK_NK + 2 * m + cp;
+          const uint4 rc = recb[i + NB * j + NF * k];
+          w[0] = rc.y & (i == 0 ? 0xffff0000u : ~0u) & (i == NB - 1 ? 0x0000ffffu : ~0u);
+          w[1] = rc.z & (j == 0 ? 0xffff0000u : ~0u) & (j == NB - 1 ? 0x0000ffffu : ~0u);
+          w[2] = rc.w & (k == 0 ? 0xffff0000u : ~0u) & (k == NB - 1 ? 0x0000ffffu : ~0u);
+        } else {
+#pragma unroll
+          for (int b = 0; b < 3; b++) w[b] = RED ? wr[m][b] : wb[m][b];
+        }
+        // keep the couplings packed across sweeps (an empty asm hides that the unpacked values
+        // of the last sweep could be reused, which would cost 12 more registers per cell)
+        asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]));
+        double* const zc = z0 + NF * (2 * m + cp);
+        double sum = half_lo(w[0]) * zc[-1];
+        sum = __builtin_fma(half_hi(w[0]), zc[1], sum);
+        sum = __builtin_fma(half_lo(w[1]), zc[-NB], sum);
+        sum = __builtin_fma(half_hi(w[1]), zc[NB], sum);
+        sum = __builtin_fma(half_lo(w[2]), zc[-NB * NB], sum);
+        sum = __builtin_fma(half_hi(w[2]), zc[NB * NB], sum);
+        const double zn = (RED ? ur[m] : ub[m]) - sum;
+        if (from_zero) {
+          zc[0] = omega * zn;
+        } else {
+          const double zo = zc[0];
+          zc[0] = __builtin_fma(omega, zn - zo, zo);
+        }
+      }
+      __syncthreads();
+    };
+    using Red = std::true_type;
+    using Black = std::false_type;
+    half(Black{}, true);
+#pragma unroll
+    for (int sweep = 1; sweep < NS; sweep++) {
+      half(Red{}, false);
+      half(Black{}, false);
+    }
+  };
+  if (REG == 1 || (REG > 1 && cls))
+    rest(std::true_type{});
+  else if constexpr (REG != 1)
+    rest(std::false_type{});
   // MUL: the stored direction is z + P e (e added to this block's values and to the ghost values
   // it pushes, which then come from z + e through every face kind)
   T* const out = (MODE == 0 ? V.pp : V.ss) + base;
@@ -616,8 +629,12 @@ __global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1
     __builtin_nontemporal_store((T)(MUL ? z[oo + NF * k] + eo : z[oo + NF * k]), out + oo + NF * k);
   T* h = MODE == 0 ? V.hpp : V.hss;
   push_halo<T, GSK_NT>(
-      B, cs[c], BC_NULL, slot, [&](int i, int j, int k) { return MUL ? z[zi(i, j, k)] + eo : z[zi(i, j, k)]; }, h,
-      h);
+      B, cs[c], BC_NULL, slot,
+      [&](int i, int j, int k) {
+        const double v = z[i + NB * (j + NB * k)];
+        return MUL ? v + eo : v;
+      },
+      h, h);
 }
 
 // Launches the sweep kernel; with the class rows (o.trec) the class-uniform variant when every
@@ -626,7 +643,10 @@ template <class T, int MODE, bool MUL>
 void launch_gsk(const BiOpts& o, hipStream_t sm, const int* active, int nact, const DevBlock* blk, const DevCase* cs,
                 const SolveState* st, BiVecs<T> V, int count, double* vs_out, const double* ce) {
   const dim3 g(nact), b(GSK_NT);
-  const int reg = !o.trec || o.nreg == 0 ? 0 : o.nirr == 0 ? 1 : 2;
+  // Three workgroups a CU, or two whose per-cell blocks are faster: with 6 % of the blocks per cell
+  // (520 blocks) P and S took 30 + 27 us against 34 + 30, with 3 % (2,480) 89 + 81 against 96 + 87, with
+  // 10 % (1,388) 60 + 55 against 56 + 50.
+  const int reg = !o.trec || o.nreg == 0 ? 0 : o.nirr == 0 ? 1 : 12 * o.nirr <= nact ? 2 : 3;
 #define GSK1(NS, R)                                                                                                 \
   hipLaunchKernelGGL((bi_precond_gsk_kernel<T, MODE, NS, MUL, R>), g, b, 0, sm, active, blk, cs, st, o.rec, V, count, \
                      vs_out, ce, o.trec, o.uni)
@@ -636,6 +656,8 @@ void launch_gsk(const BiOpts& o, hipStream_t sm, const int* active, int nact, co
       GSK1(NS, 1);         \
     else if (reg == 2)     \
       GSK1(NS, 2);         \
+    else if (reg == 3)     \
+      GSK1(NS, 3);         \
     else                   \
       GSK1(NS, 0);         \
   } while (0)

@@ -64,13 +64,6 @@ struct PutDevice {
   }
 };
 
-// a or b by value: the conditional operator on two array elements selects an address, which would put
-// the arrays in memory
-template <class T>
-__device__ inline T pick(bool c, T a, T b) {
-  return c ? a : b;
-}
-
 // a value that every lane has, in scalar registers (a struct of 8-byte and 4-byte members too)
 template <class V>
 __device__ inline V scalar(V v) {
