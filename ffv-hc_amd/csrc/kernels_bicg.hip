@@ -99,6 +99,29 @@ __global__ __launch_bounds__(BI_NT) void bi_init_kernel(const int* __restrict__ 
   }
 }
 
+// Vectors that a kernel streams through once.  Where the solve's eight vectors do not fit the 256 MB
+// last-level cache (streams(): more than 1,024 blocks of FP64), non-temporal accesses leave it to what the
+// next kernels read: the FP64 matvecs after P and S take 46 / 48 us instead of 60 / 57 at 2,480 blocks and
+// 28 / 31 instead of 30 / 33 at 1,388.  Where they fit, plain ones keep them there: at 520 blocks the
+// matvecs after the sweeps take 11.1 us instead of 12.5, the FP64 P and S 19.8 and 16.7 instead of 21.9
+// and 19.3.
+template <class T>
+inline bool streams(int nact) {
+  return (size_t)nact * NC * sizeof(T) * 8 > (size_t)256 << 20;
+}
+template <bool NT, class T>
+__device__ inline T load_stream(const T* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  return *p;
+}
+template <bool NT, class T>
+__device__ inline void store_stream(T v, T* p) {
+  if constexpr (NT)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+
 // P: p update and p_ = M p with its ghost layer (mode 0); S: s = r - alpha q_, s_ = M s (mode 1)
 // TA: storage precision of the matrix (FP32 copies for an FP64 solve are widened on load)
 template <class T, int MODE, class TA = T>
@@ -106,7 +129,7 @@ __global__ __launch_bounds__(BI_NT) void bi_precond_kernel(const int* __restrict
                                                            const DevBlock* __restrict__ blk,
                                                            const DevCase* __restrict__ cs,
                                                            const SolveState* __restrict__ st, Coef7<TA> A, BiVecs<T> V,
-                                                           int count, ClassRows<TA> R) {
+                                                           int count, ClassRows<TA> R, int nt) {
   __shared__ T s[LP * LP * LP];
   const int slot = active[blockIdx.x];
   const DevBlock& B = blk[slot];
@@ -120,44 +143,50 @@ __global__ __launch_bounds__(BI_NT) void bi_precond_kernel(const int* __restrict
   // arguments); FIN_BI_XR of the previous iteration stored it in iter
   const bool first = (count > 0 ? count : st[c].iter + 1) == 1 || st[c].restart;
   constexpr int KB = Batch<T>::K;
-  by_class(R, slot, [&](auto cls) {
-    constexpr bool CLS = decltype(cls)::value;
-    const TA* tr = CLS ? class_column(R.tab, slot, tx, ty) : nullptr;
-    const T alo = CLS ? (T)tr[0] : (T)0, ain = CLS ? (T)tr[9 * 8] : (T)0, ahi = CLS ? (T)tr[18 * 8] : (T)0;
+  auto form = [&](auto nt_tag) __attribute__((always_inline)) {
+    constexpr bool NT = decltype(nt_tag)::value;
+    by_class(R, slot, [&](auto cls) {
+      constexpr bool CLS = decltype(cls)::value;
+      const TA* tr = CLS ? class_column(R.tab, slot, tx, ty) : nullptr;
+      const T alo = CLS ? (T)tr[0] : (T)0, ain = CLS ? (T)tr[9 * 8] : (T)0, ahi = CLS ? (T)tr[18 * 8] : (T)0;
 #pragma unroll
-    for (int k0 = 0; k0 < NB; k0 += KB) {
-      T rv[KB], pv[KB], qv[KB], ap[KB];
+      for (int k0 = 0; k0 < NB; k0 += KB) {
+        T rv[KB], pv[KB], qv[KB], ap[KB];
 #pragma unroll
-      for (int kk = 0; kk < KB; kk++) {
-        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-        rv[kk] = V.r[g];
-        ap[kk] = CLS ? (k0 + kk == 0 ? alo : k0 + kk == NB - 1 ? ahi : ain) : (T)A.p[0][g];
-        if (MODE == 1 || !first) qv[kk] = V.q[g];
-        if (MODE == 0 && !first) pv[kk] = V.p[g];
-      }
-#pragma unroll
-      for (int kk = 0; kk < KB; kk++) {
-        const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
-        T v;
-        if (MODE == 0) {
-          if (first) {
-            v = rv[kk];
-          } else {
-            const T tmp = pv[kk] + ng * qv[kk];  // AXPY(p, q_, -gamma)
-            v = rv[kk] + beta * tmp;             // XPAY(p, r, beta)
-          }
-          V.p[g] = v;
-        } else {
-          v = na * qv[kk] + rv[kk];  // AXPYZ(s, q_, r, -alpha)
-          V.s[g] = v;
+        for (int kk = 0; kk < KB; kk++) {
+          const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+          rv[kk] = load_stream<NT>(V.r + g);
+          ap[kk] = CLS ? (k0 + kk == 0 ? alo : k0 + kk == NB - 1 ? ahi : ain) : (T)A.p[0][g];
+          if (MODE == 1 || !first) qv[kk] = load_stream<NT>(V.q + g);
+          if (MODE == 0 && !first) pv[kk] = load_stream<NT>(V.p + g);
         }
-        const T m = omega * (v / ap[kk]);
-        if (MODE == 0) V.pp[g] = m;
-        else V.ss[g] = m;
-        s[lds(tx, ty, k0 + kk)] = m;
+#pragma unroll
+        for (int kk = 0; kk < KB; kk++) {
+          const size_t g = base + tx + NB * (ty + NB * (k0 + kk));
+          T v;
+          if (MODE == 0) {
+            if (first) {
+              v = rv[kk];
+            } else {
+              const T tmp = pv[kk] + ng * qv[kk];  // AXPY(p, q_, -gamma)
+              v = rv[kk] + beta * tmp;             // XPAY(p, r, beta)
+            }
+            store_stream<NT>(v, V.p + g);
+          } else {
+            v = na * qv[kk] + rv[kk];  // AXPYZ(s, q_, r, -alpha)
+            store_stream<NT>(v, V.s + g);
+          }
+          const T m = omega * (v / ap[kk]);
+          store_stream<NT>(m, (MODE == 0 ? V.pp : V.ss) + g);
+          s[lds(tx, ty, k0 + kk)] = m;
+        }
       }
-    }
-  });
+    });
+  };
+  if (nt)
+    form(std::true_type{});
+  else
+    form(std::false_type{});
   __syncthreads();
   T* h = MODE == 0 ? V.hpp : V.hss;
   push_halo<T, BI_NT>(B, cs[c], BC_NULL, slot, [&](int i, int j, int k) { return s[lds(i, j, k)]; }, h, h);
@@ -420,7 +449,7 @@ __global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1
     const int* __restrict__ active, const DevBlock* __restrict__ blk, const DevCase* __restrict__ cs,
     const SolveState* __restrict__ st, const uint4* __restrict__ rec, BiVecs<T> V, int count,
     double* __restrict__ vs_out, const double* __restrict__ ce, const uint4* __restrict__ trec,
-    const int* __restrict__ uni) {
+    const int* __restrict__ uni, int nt) {
   __shared__ double zpad[NC + 2 * NF];  // z with a zero plane below (k = -1) and above (k = NB)
   __shared__ double red[GSK_NT / 64];
   const int slot = active[blockIdx.x];
@@ -499,7 +528,8 @@ __global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1
       for (int kk = 0; kk < KB; kk++) {
         const unsigned o = o0 + NF * (k0 + kk);
         // streamed once through this kernel: non-temporal loads and stores leave the caches to what
-        // the next kernels read (measured: this kernel 3% faster, the matvecs after it 3-7%)
+        // the next kernels read (measured: this kernel 3% faster, the matvecs after it 3-7%; the result
+        // is stored so only where the vectors do not fit, streams())
         rv[kk] = __builtin_nontemporal_load(rb + o);
         if (MODE == 1 || !first) qv[kk] = __builtin_nontemporal_load(qb + o);
         if (MODE == 0 && !first) pv[kk] = __builtin_nontemporal_load(vb + o);
@@ -624,9 +654,15 @@ __global__ __launch_bounds__(GSK_NT) __attribute__((amdgpu_waves_per_eu(REG == 1
   T* const out = (MODE == 0 ? V.pp : V.ss) + base;
   unsigned oo = o0;  // opaque: the store offsets are formed here, not held across the sweeps
   asm volatile("" : "+v"(oo));
+  auto put = [&](auto nt_tag) __attribute__((always_inline)) {
 #pragma unroll
-  for (int k = 0; k < GSK_NK; k++)
-    __builtin_nontemporal_store((T)(MUL ? z[oo + NF * k] + eo : z[oo + NF * k]), out + oo + NF * k);
+    for (int k = 0; k < GSK_NK; k++)
+      store_stream<decltype(nt_tag)::value>((T)(MUL ? z[oo + NF * k] + eo : z[oo + NF * k]), out + oo + NF * k);
+  };
+  if (nt)
+    put(std::true_type{});
+  else
+    put(std::false_type{});
   T* h = MODE == 0 ? V.hpp : V.hss;
   push_halo<T, GSK_NT>(
       B, cs[c], BC_NULL, slot,
@@ -649,7 +685,7 @@ void launch_gsk(const BiOpts& o, hipStream_t sm, const int* active, int nact, co
   const int reg = !o.trec || o.nreg == 0 ? 0 : o.nirr == 0 ? 1 : 12 * o.nirr <= nact ? 2 : 3;
 #define GSK1(NS, R)                                                                                                 \
   hipLaunchKernelGGL((bi_precond_gsk_kernel<T, MODE, NS, MUL, R>), g, b, 0, sm, active, blk, cs, st, o.rec, V, count, \
-                     vs_out, ce, o.trec, o.uni)
+                     vs_out, ce, o.trec, o.uni, (int)streams<T>(nact))
 #define GSK(NS)            \
   do {                     \
     if (reg == 1)          \
@@ -1050,10 +1086,10 @@ void launch_bicgstab_iter(hipStream_t sm, const int* active, int nact, const int
                          *o.M64, Vd, count);
     else if (dbl && o.A32)
       hipLaunchKernelGGL((bi_precond_kernel<double, MODE, float>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs,
-                         st, *o.A32, Vd, count, ClassRows<float>());
+                         st, *o.A32, Vd, count, ClassRows<float>(), 0);
     else
       hipLaunchKernelGGL((bi_precond_kernel<T, MODE>), dim3(nact), dim3(BI_NT), 0, sm, active, blk, cs, st, A, V,
-                         count, R);
+                         count, R, (int)streams<T>(nact));
   };
   // the T stage keeps its partials in part[2..3] (XR reads them while writing part[0..1])
   auto matvec = [&](auto mode_tag) {
