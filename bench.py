@@ -347,6 +347,13 @@ STEP_FIXED_BYTES_IMPLICIT_U = 3 * 180 + 164 + 212 + 236 + 144
 DEFECT_BYTES = 80
 
 
+def fp64_iteration_bytes(uniform):
+    """Bytes per cell of an FP64 Jacobi-BiCGSTAB iteration of the step: the class-uniform blocks (a
+    fraction `uniform`) read 27 rows in place of P's and S's diagonal and Q's and T's seven bands.  (A
+    resident solve, of at most 512 blocks, keeps its vectors on the chip and moves less.)"""
+    return step_iteration_bytes(None, 0.0) - uniform * (1 + 7 + 1 + 7) * 8
+
+
 def step_iteration_bytes(method, uniform_fraction):
     """Bytes per cell of one Krylov iteration of the pressure solve: the reference's FP64 Jacobi-
     BiCGSTAB (method None) or solve_mixed `method`, whose class-uniform blocks read 27 rows instead
@@ -578,12 +585,13 @@ def time_step_leg(case, steps, warmup, method, omega, fp64_steps=None):
         st = ctx.stats(F.ux, ncases=1)[0]
         nu, no = ctx.stencil_classes(F.A)
         m = None if tag == "fp64" else method
-        per_it = step_iteration_bytes(m, nu / max(nu + no, 1))
+        uniform = nu / max(nu + no, 1)
+        per_it = fp64_iteration_bytes(uniform) if m is None else step_iteration_bytes(m, uniform)
         mean_it = float(np.mean(its))
         mean_uit = float(np.mean(uits))
         coarse = 0.0 if m is None or m < 17 else 2 * 4.0 * tree.nblk * ((tree.nblk + 3) // 4 * 4) * mean_it
         fixed = STEP_FIXED_BYTES_IMPLICIT_U if implicit else STEP_FIXED_BYTES
-        step_bytes = (fixed + mean_it * per_it + mean_uit * step_iteration_bytes(None, 0.0) +
+        step_bytes = (fixed + mean_it * per_it + mean_uit * fp64_iteration_bytes(uniform) +
                       (0 if m is None else DEFECT_BYTES)) * cells + coarse
         gbs = step_bytes * nsteps / dt / 1e9
         out[tag] = {"steps": nsteps, "ms_per_step": round(dt / nsteps * 1e3, 3),
