@@ -27,8 +27,8 @@
 //
 // The arithmetic, each sum's order included, is that of the launch-per-stage kernels: the same bits.
 //
-// Measured, one iteration with one launch per stage -> resident: two-level BiCGSTAB 55 -> 32 us at 128
-// blocks (of 32: two preconditioners 2 x 8, meetings 13), Jacobi BiCGSTAB 46 -> 21 us at 128 and 68 ->
+// Measured, one iteration with one launch per stage -> resident: two-level BiCGSTAB 55 -> 30 us at 128
+// blocks (two preconditioners 2 x 8, meetings 13), Jacobi BiCGSTAB 46 -> 20 us at 128 and 68 ->
 // 28 us at 256 blocks, PCG 26 -> 10 us at 60, RBGS 14 -> 8.6 us and Jacobi 13.4 -> 7.9 us at 128.  A
 // meeting of everyone takes 2.4 us with 16 workgroups and 3.4-4 with 128, one of neighbours 1.4-2.
 // PAIR, a solve: Jacobi BiCGSTAB 48.5 -> 25.7 ms at 288 and 59.7 -> 32.7 ms at 512 blocks, PCG 35.4 -> 20.9
