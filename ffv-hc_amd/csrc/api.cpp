@@ -160,14 +160,33 @@ static void make_case_meta(ffvhc_ctx* c, int id) {
   c->pcase[id] = d;
 }
 
+// A context of one case should not pay for a thousand: 64 cases' room at first (a page-locked allocation
+// costs 0.2 ms and more with its size), twice the need after that.
+int pinned_cases(ffvhc_ctx* c, size_t n) {
+  if (n <= c->pcases) return 0;
+  HIPCHK(hipStreamSynchronize(c->sm));  // a copy may still read or write the old one
+  const size_t k = std::max<size_t>(64, 2 * n);
+  c->pcases = 0;
+  HIPCHK(c->parena.reserve(k * (sizeof(DevCase) + sizeof(SolveState) + 5 * sizeof(double))));
+  c->presult = reinterpret_cast<double*>(c->parena.data());
+  c->pst = reinterpret_cast<SolveState*>(c->presult + 5 * k);
+  c->pcase = reinterpret_cast<DevCase*>(c->pst + k);
+  c->pcases = k;
+  return 0;
+}
+
 // One copy per run of consecutive ids, in selection order; the entries are read from pinned memory while the
 // stream runs, so a caller that does not wait before it returns must not be followed by another change.
 int send_case_meta(ffvhc_ctx* c, const std::vector<int>& ids) {
+  for (int id : ids) {
+    int rc = pinned_cases(c, (size_t)id + 1);
+    if (rc) return rc;
+  }
   for (size_t i = 0; i < ids.size();) {
     size_t e = i;
     do make_case_meta(c, ids[e++]);
     while (e < ids.size() && ids[e] == ids[e - 1] + 1);
-    HIPCHK(hipMemcpyAsync(c->dcase + ids[i], c->pcase.data() + ids[i], sizeof(DevCase) * (e - i), hipMemcpyHostToDevice,
+    HIPCHK(hipMemcpyAsync(c->dcase + ids[i], c->pcase + ids[i], sizeof(DevCase) * (e - i), hipMemcpyHostToDevice,
                           c->sm));
     i = e;
   }
@@ -298,10 +317,6 @@ int ffvhc_ctx_create(int device, long long max_blocks, ffvhc_ctx** out) {
   c->hst.assign(MAX_CASES, SolveState{});
   c->hst2.assign(MAX_CASES, SolveState{});
   c->fields.reserve(MAX_FIELDS);
-  HIPCHK(c->pcase.reserve(MAX_CASES));
-  HIPCHK(c->pst.reserve(MAX_CASES));
-  HIPCHK(c->presult.reserve(5 * (size_t)MAX_CASES));
-  for (auto& e : c->ev_step) HIPCHK(hipEventCreate(&e));
   HIPCHK(hipMalloc(&c->dblk, sizeof(DevBlock) * max_blocks));
   HIPCHK(hipMalloc(&c->dcase, sizeof(DevCase) * MAX_CASES));
   HIPCHK(hipMalloc(&c->dactive, sizeof(int) * max_blocks));
@@ -359,7 +374,8 @@ void ffvhc_ctx_destroy(ffvhc_ctx* c) {
   (void)hipFree(c->dflag);
   (void)hipFree(c->dcid);
   if (c->blas) (void)rocblas_destroy_handle((rocblas_handle)c->blas);
-  for (auto& e : c->ev_step) (void)hipEventDestroy(e);
+  for (auto& e : c->ev_step)
+    if (e) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(c->sm);
   if (c->sc) {
     (void)hipEventDestroy(c->ev_cs);

@@ -853,7 +853,6 @@ __global__ __launch_bounds__(RS_NT, PAIR ? 4 : 2) void resident_cg_kernel(Reside
   if (S.done) return;
   const DevCase& C = a.cs[c];
   const int t = threadIdx.x, tx = t & 15, ty = (t >> 4) & 15, kb = (t >> 8) * RS_NK, lane = t & 63;
-  const bool lower = kb == 0;
   const size_t g0 = (size_t)slot * NC + tx + NB * ty + NF * kb;
   Meeting meet{a.words, a.nslots, C.slot_begin, C.nblk, slot};
   if (t == 0) {

@@ -84,10 +84,14 @@ struct ffvhc_ctx {
   std::vector<ffvhc::DevBlock> hblk;
   ffvhc::DevBlock* dblk = nullptr;
   std::vector<ffvhc::DevCase> hcase;
-  ffvhc::Pinned<ffvhc::DevCase> pcase;       // hcase as last sent to dcase
-  ffvhc::Pinned<ffvhc::SolveState> pst;      // where the states of a solve are read back
-  ffvhc::Pinned<double> presult;             // where kernels write per-case results
-  hipEvent_t ev_step[4] = {};                // the stages of ffvhc_step
+  // one page-locked allocation for pcases cases (pinned_cases): hcase as last sent to dcase, where the
+  // states of a solve are read back, and where kernels write five results per case
+  ffvhc::Pinned<char> parena;
+  size_t pcases = 0;
+  ffvhc::DevCase* pcase = nullptr;
+  ffvhc::SolveState* pst = nullptr;
+  double* presult = nullptr;
+  hipEvent_t ev_step[4] = {};  // the stages of ffvhc_step, made by its first call
   ffvhc::DevCase* dcase = nullptr;
   std::vector<ffvhc::CaseRec> cases;
   // geometry per slot: cut distances (float, exact: Cutlib stores float32), cell flags
@@ -213,5 +217,6 @@ int scratch_field(ffvhc_ctx* ctx, int prec, int role, int* field);
 bool field_ok(ffvhc_ctx* ctx, int f, int prec);
 int upload_case_meta(ffvhc_ctx* c, int id);
 int send_case_meta(ffvhc_ctx* c, const std::vector<int>& ids);  // without waiting
+int pinned_cases(ffvhc_ctx* c, size_t n);  // room for n cases in the page-locked buffers
 int host_impose_bc(ffvhc_ctx* c, int id, double* padded, int g, int bcg, int updater);
 }  // namespace ffvhc

@@ -50,9 +50,11 @@ Coef7<T> coef(ffvhc_ctx* c, const int* A) {
 
 int sync_state(ffvhc_ctx* c, SolveState* dst, std::vector<SolveState>& hst) {
   const size_t n = c->cases.size();
-  HIPCHK(hipMemcpyAsync(c->pst.data(), dst, sizeof(SolveState) * n, hipMemcpyDeviceToHost, c->sm));
+  int rc = pinned_cases(c, n);
+  if (rc) return rc;
+  HIPCHK(hipMemcpyAsync(c->pst, dst, sizeof(SolveState) * n, hipMemcpyDeviceToHost, c->sm));
   HIPCHK(hipStreamSynchronize(c->sm));
-  std::copy(c->pst.data(), c->pst.data() + n, hst.begin());
+  std::copy(c->pst, c->pst + n, hst.begin());
   return 0;
 }
 
@@ -1637,9 +1639,11 @@ static int case_triples(ffvhc_ctx* c, double* f, Launch launch) {
   int rc = refresh_active(c);
   if (rc) return rc;
   // the kernel writes the triples to the host (a device buffer and a copy back took 12 us more)
-  const double* const h = c->presult.data();
+  rc = pinned_cases(c, (size_t)c->ncaseact);
+  if (rc) return rc;
+  const double* const h = c->presult;
   void* dout = nullptr;
-  HIPCHK(hipHostGetDevicePointer(&dout, c->presult.data(), 0));
+  if (h) HIPCHK(hipHostGetDevicePointer(&dout, c->presult, 0));
   launch((double*)dout);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->sm));
@@ -1732,9 +1736,11 @@ int ffvhc_field_stats(ffvhc_ctx* c, int f, double* out) {
   int rc = refresh_active(c);
   if (rc) return rc;
   const std::vector<int> ids = selected_cases(c);
-  const double* const h = c->presult.data();
+  rc = pinned_cases(c, (size_t)c->ncaseact);
+  if (rc) return rc;
+  const double* const h = c->presult;
   void* dout = nullptr;
-  HIPCHK(hipHostGetDevicePointer(&dout, c->presult.data(), 0));
+  if (h) HIPCHK(hipHostGetDevicePointer(&dout, c->presult, 0));
   launch_stats(c->sm, c->dactive, c->nactive, c->dcaseact, c->ncaseact, c->dcase, (const double*)c->fields[f].d[0],
                c->dpart, (size_t)c->cap, (double*)dout);
   HIPCHK(hipGetLastError());
@@ -1833,6 +1839,8 @@ int ffvhc_step(ffvhc_ctx* c, ffvhc_step_fields* F, const ffvhc_step_params* P, f
     launch_ghost_pull<double>(c->sm, c->dactive, c->nactive, c->dblk, c->dcase, G, c->multilevel);
   };
   hipEvent_t(&ev)[4] = c->ev_step;
+  for (auto& e : ev)
+    if (!e) HIPCHK(hipEventCreate(&e));
   HIPCHK(hipEventRecord(ev[0], c->sm));
   const size_t nc = ids.size();
   std::vector<int> cntu(3 * nc, 0);

@@ -76,3 +76,23 @@ def test_parameters_of_selected_cases(ids):
         assert len({together[q].tobytes() for q in ids}) == len(ids)
     finally:
         ctx.close()
+
+
+def test_results_of_many_cases():
+    """More cases than the page-locked buffers hold at first: parameters, statistics and solves of each."""
+    tree = ffvhc.Tree(root=(1, 1, 1), root_length=1.0)
+    ctx = ffvhc.Context(max_blocks=150)
+    try:
+        f = ctx.field(8)
+        cids = []
+        for q in range(150):
+            cids.append(ctx.add_case(tree, ffvhc.case_params(dt=0.001 * (1 + q), bc=BC)))
+            ctx.upload(f, cids[-1], np.full((1,) + (N + 2 * G,) * 3, 1.0 + q))
+            if q in (63, 64, 149):
+                ctx.select(cids)
+                assert [s[1] for s in ctx.stats(f, ncases=q + 1)] == [1.0 + c for c in range(q + 1)]
+                cfl, _ = ctx.cfl(f, ncases=q + 1)
+                want = [(1.0 + c) * 0.001 * (1 + c) / 1.0 for c in range(q + 1)]
+                assert np.allclose(cfl, want, rtol=1e-14, atol=0.0)
+    finally:
+        ctx.close()
